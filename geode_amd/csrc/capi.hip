@@ -294,10 +294,10 @@ int ffn_swiglu_ws(const gv_q4 *gate, const gv_q4 *up, const gv_q4 *down, int M, 
     _Float16 *act = reinterpret_cast<_Float16 *>(m + static_cast<size_t>(M) * F);
     hipStream_t st = stream();
     const int64_t ab_h = act_halves(H), ab_f = act_halves(F);
-    int waves = 0, kw = 0;
-    if (M <= 8 && F % 16 == 0 && H <= 8192 && mfma_split(H, 1, waves, kw) && waves <= 4) {
-        // three launches: x's operands (in x's place: M act rows of H fit its M x H floats), gate | up with the
-        // SwiGLU and its quantization (act), down
+    if (H <= 8192 && (M <= 8 || F <= 8192) && ffn_up_fits(to_q4(*gate), to_q4(*up), M)) {
+        // x's operands (in x's place: M act rows of H fit its M x H floats), gate | up with the SwiGLU and its
+        // quantization (act), down. Wider inputs than the gate | up launch's eight waves take go on below, in a launch
+        // a phase (17 rows of 2048 -> 6144: 58 us a call that way, 30 this one).
         _Float16 *act_x = reinterpret_cast<_Float16 *>(x);
         if (quantize_f16(x_f16, M, static_cast<int>(H), act_x, ab_h, st) != 0) return -1;
         if (ffn_up(to_q4(*gate), to_q4(*up), act_x, ab_h, M, act, ab_f, st) != 0) return -1;

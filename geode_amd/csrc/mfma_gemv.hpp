@@ -270,6 +270,22 @@ struct TileRun {
     int64_t t0;
     __device__ int64_t operator()(int i) const { return t0 + i; }
 };
+// The matrix a call's tiles come from: one matrix's codes and scales, or a pair's (local tile i from the first where i
+// is even, from the second where it is odd: a gate and an up matrix of the same shape, their tiles in turns)
+struct OneMatrix {
+    const uint8_t *codes_, *scales_;
+    __device__ OneMatrix at(int64_t co, int64_t so) const { return OneMatrix{codes_ + co, scales_ + so}; }
+    __device__ const uint8_t *codes(int) const { return codes_; }
+    __device__ const uint8_t *scales(int) const { return scales_; }
+};
+struct MatrixPair {
+    const uint8_t *codes0, *scales0, *codes1, *scales1;
+    __device__ MatrixPair at(int64_t co, int64_t so) const {
+        return MatrixPair{codes0 + co, scales0 + so, codes1 + co, scales1 + so};
+    }
+    __device__ const uint8_t *codes(int i) const { return (i & 1) ? codes1 : codes0; }
+    __device__ const uint8_t *scales(int i) const { return (i & 1) ? scales1 : scales0; }
+};
 struct NoHook {
     __device__ void operator()() const {}
 };
@@ -309,11 +325,10 @@ enum TilesMode { kSplitK = 0, kKeepParts = 1, kWaveTiles = 2 };
 // the activations and the first tiles are in registers. Every thread of the workgroup calls this.
 template <int KW, int NTT, int MODE, int NT = 0, int DEPTH = 3, bool PACK = false, int FLUSH = 0, typename RowFn,
           typename PutFn, typename MapFn = TileRun, typename HookFn = NoHook, typename ReadyFn = NoHook,
-          typename FlushFn = NoFlush>
-__device__ inline void mfma_tiles(const uint8_t *__restrict__ codes, const uint8_t *__restrict__ scales, int64_t rows,
-                                  int nsc, int sc0, int nt, int M, RowFn rowp, PutFn put, f4 *part, uint2 *tab,
-                                  MapFn tmap, HookFn hook = HookFn{}, ReadyFn ready = ReadyFn{},
-                                  FlushFn flush = FlushFn{}) {
+          typename FlushFn = NoFlush, typename MatFn = OneMatrix>
+__device__ inline void mfma_tiles_of(const MatFn mat, int64_t rows, int nsc, int sc0, int nt, int M, RowFn rowp,
+                                     PutFn put, f4 *part, uint2 *tab, MapFn tmap, HookFn hook = HookFn{},
+                                     ReadyFn ready = ReadyFn{}, FlushFn flush = FlushFn{}) {
     static_assert(DEPTH >= 2 && (NT > 0 || DEPTH >= 3), "the runtime loop is a ring of at least three");
     static_assert(!PACK || NTT == 1, "packed hi | lo columns take one 16-row tile of at most 8 rows");
     static_assert(FLUSH == 0 || (MODE == kSplitK && NT == 0), "the flushed split-K runs the runtime tile loop");
@@ -323,17 +338,18 @@ __device__ inline void mfma_tiles(const uint8_t *__restrict__ codes, const uint8
     const int l = threadIdx.x % 64, lq = l % 16, lg = l / 16;
     constexpr int NS = KW / 4;   // super-chunks a wave takes
     const uint32_t magic = 0x64006400u;
-    const uint8_t *cbase = codes + static_cast<int64_t>(sc0 + w * NS) * 1024 + l * 16;
     // the lane's scale words of its NS super-chunks: adjacent in one quad (sc0 a multiple of 4, NS = 1, 2 or 4)
     const uint32_t nsq_u = static_cast<uint32_t>((nsc + 3) / 4);
-    const uint8_t *sbase =
-        scales + static_cast<int64_t>((sc0 + w * NS) / 4) * 512 + ((lq * 2 + lg / 2) * 4 + (sc0 + w * NS) % 4) * 4;
+    const MatFn base = mat.at(static_cast<int64_t>(sc0 + w * NS) * 1024 + l * 16,
+                              static_cast<int64_t>((sc0 + w * NS) / 4) * 512 +
+                                  ((lq * 2 + lg / 2) * 4 + (sc0 + w * NS) % 4) * 4);
     // Every load is issued unconditionally (a tile past nt reads the last tile again, from the cache): a branch
     // around a load makes the compiler wait for nearly all loads in flight before the next use. Offsets in 32 bits
     // (a matrix < 4 GB).
     const uint32_t nsc_u = static_cast<uint32_t>(nsc);
     auto load = [&](int i, uint4 (&cw)[NS], uint32_t (&sw)[NS]) {
         const uint32_t T = nt > 0 ? static_cast<uint32_t>(tmap(i < nt ? i : nt - 1)) : 0u;
+        const uint8_t *cbase = base.codes(i), *sbase = base.scales(i);
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
             const uint32_t blk = T * nsc_u + static_cast<uint32_t>(s);
@@ -387,24 +403,31 @@ __device__ inline void mfma_tiles(const uint8_t *__restrict__ codes, const uint8
         for (int tt = 0; tt < NTT; ++tt)
 #pragma unroll
             for (int h = 0; h < NB; ++h) acc[h][tt] = f4{0, 0, 0, 0};
-        uint2 tv[NS][4];   // the tile's scale table entries, all read from the LDS before the first is used
+        // the tile's scale table entries, all read from the LDS before the first is used (a call of one tile: two
+        // super-chunks' at a time, which keeps twelve waves of sixteen chunks within their registers)
+        constexpr int NV = NT == 1 && NS == 4 ? 2 : NS;
 #pragma unroll
-        for (int s = 0; s < NS; ++s)
+        for (int s0 = 0; s0 < NS; s0 += NV) {
+            uint2 tv[NV][4];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) tv[s][j] = tab[(sq[s] >> (8 * j)) & 0xFFu];
-        __builtin_amdgcn_sched_barrier(0);
+            for (int s = 0; s < NV; ++s)
 #pragma unroll
-        for (int s = 0; s < NS; ++s) {
-            const uint32_t words[4] = {cq[s].x, cq[s].y, cq[s].z, cq[s].w};
+                for (int j = 0; j < 4; ++j) tv[s][j] = tab[(sq[s0 + s] >> (8 * j)) & 0xFFu];
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const h8 a = decode8(words[j], tv[s][j], magic);
-                const int c = s * 4 + j;
+            for (int s = 0; s < NV; ++s) {
+                const uint4 &cs = cq[s0 + s];
+                const uint32_t words[4] = {cs.x, cs.y, cs.z, cs.w};
 #pragma unroll
-                for (int tt = 0; tt < NTT; ++tt)
+                for (int j = 0; j < 4; ++j) {
+                    const h8 a = decode8(words[j], tv[s][j], magic);
+                    const int c = (s0 + s) * 4 + j;
 #pragma unroll
-                    for (int h = 0; h < NB; ++h)
-                        acc[h][tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b[h][c][tt], acc[h][tt], 0, 0, 0);
+                    for (int tt = 0; tt < NTT; ++tt)
+#pragma unroll
+                        for (int h = 0; h < NB; ++h)
+                            acc[h][tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b[h][c][tt], acc[h][tt], 0, 0, 0);
+                }
             }
         }
 #pragma unroll
@@ -491,6 +514,69 @@ __device__ inline void mfma_tiles(const uint8_t *__restrict__ codes, const uint8
         return;
     }
     if (MODE == kSplitK && FLUSH == 0) split_k_out(0, nt);
+}
+
+// mfma_tiles_of over one matrix
+template <int KW, int NTT, int MODE, int NT = 0, int DEPTH = 3, bool PACK = false, int FLUSH = 0, typename RowFn,
+          typename PutFn, typename MapFn = TileRun, typename HookFn = NoHook, typename ReadyFn = NoHook,
+          typename FlushFn = NoFlush>
+__device__ inline void mfma_tiles(const uint8_t *__restrict__ codes, const uint8_t *__restrict__ scales, int64_t rows,
+                                  int nsc, int sc0, int nt, int M, RowFn rowp, PutFn put, f4 *part, uint2 *tab,
+                                  MapFn tmap, HookFn hook = HookFn{}, ReadyFn ready = ReadyFn{},
+                                  FlushFn flush = FlushFn{}) {
+    mfma_tiles_of<KW, NTT, MODE, NT, DEPTH, PACK, FLUSH>(OneMatrix{codes, scales}, rows, nsc, sc0, nt, M, rowp, put,
+                                                         part, tab, tmap, hook, ready, flush);
+}
+
+// The SwiGLU of a matched gate / up tile pair's sums for F tile p (gs, us: the lane's rows 4 lg .. 4 lg + 3 of its
+// column; x their globals g0, g1), m = silu(gate) x up (kernels.hpp:141), quantized per 16-value
+// block (the pair's 16 rows: the column's four lanes) into the act16 operands of the column's row (live: the column
+// is a pick). Every lane of the wave calls it (lane shuffles).
+__device__ inline void swiglu_pair_out(f4 gs, f4 us, float g0, float g1, int p, bool live, _Float16 *row) {
+    const int lg = (threadIdx.x % 64) / 16;
+    float mv[4], amax = 0.0f;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const float x = gs[r] * g0, uv = us[r] * g1;
+        mv[r] = __fmul_rn(__fdiv_rn(x, __fadd_rn(1.0f, expf(-x))), uv);
+        amax = fmaxf(amax, fabsf(mv[r]));
+    }
+    amax = fmaxf(amax, __shfl_xor(amax, 16, 64));
+    amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
+    const float sc = __fdiv_rn(amax, 127.0f), qi = amax > 0.0f ? __fdiv_rn(127.0f, amax) : 0.0f;
+    uint32_t hw[2], lw[2];   // this lane's 4 values (rows 4 lg .. 4 lg + 3 of the pair): hi, lo halves
+#pragma unroll
+    for (int r = 0; r < 4; r += 2) {
+        _Float16 h0, l0, h1, l1;
+        const int q0 = min(max(static_cast<int>(rintf(__fmul_rn(mv[r], qi))), -127), 127);
+        const int q1 = min(max(static_cast<int>(rintf(__fmul_rn(mv[r + 1], qi))), -127), 127);
+        const bool ex = g_act_exact != 0;   // (the exact path: the SwiGLU values themselves)
+        split_f16(ex ? mv[r] : __fmul_rn(static_cast<float>(q0), sc), h0, l0);
+        split_f16(ex ? mv[r + 1] : __fmul_rn(static_cast<float>(q1), sc), h1, l1);
+        hw[r / 2] = static_cast<uint32_t>(__builtin_bit_cast(uint16_t, h0)) |
+                    (static_cast<uint32_t>(__builtin_bit_cast(uint16_t, h1)) << 16);
+        lw[r / 2] = static_cast<uint32_t>(__builtin_bit_cast(uint16_t, l0)) |
+                    (static_cast<uint32_t>(__builtin_bit_cast(uint16_t, l1)) << 16);
+    }
+    // k-group 2 p + lg / 2 holds values 0..3 (lane lg even) and 4..7 (lane lg + 1) in the slot order
+    // (0 4 1 5 2 6 3 7): the even lane takes its partner's four and writes the group
+    uint32_t ph[2], pl[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        ph[k] = __shfl_xor(hw[k], 16, 64);
+        pl[k] = __shfl_xor(lw[k], 16, 64);
+    }
+    if ((lg & 1) == 0 && live) {
+        auto inter = [](uint32_t mine, uint32_t other) {   // (m0, o0), (m1, o1) as two words
+            return make_uint2((mine & 0xFFFFu) | (other << 16), (mine >> 16) | (other & 0xFFFF0000u));
+        };
+        const uint2 h01 = inter(hw[0], ph[0]), h23 = inter(hw[1], ph[1]);
+        const uint2 l01 = inter(lw[0], pl[0]), l23 = inter(lw[1], pl[1]);
+        const int gi = 2 * p + lg / 2;
+        uint4 *dst = reinterpret_cast<uint4 *>(row + static_cast<int64_t>(gi) * 16);
+        dst[0] = make_uint4(h01.x, h01.y, h23.x, h23.y);
+        dst[1] = make_uint4(l01.x, l01.y, l23.x, l23.y);
+    }
 }
 
 }  // namespace gv

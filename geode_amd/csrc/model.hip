@@ -919,57 +919,6 @@ __global__ __launch_bounds__(512) void mixout_kernel(const MixOutArgs a) {
 // slot's rows once) and the chip ends the launch together.
 constexpr int kMoeFlush = 8;   // tiles whose partial sums an expert workgroup holds at once
 
-// The SwiGLU of a matched gate / up tile pair's sums for F tile p (gs, us: the lane's rows 4 lg .. 4 lg + 3 of its
-// column; x their globals g0, g1), m = silu(gate) x up (swiglu_quant_kernel's arithmetic), quantized per 16-value
-// block (the pair's 16 rows: the column's four lanes) into the act16 operands of the column's row (live: the column
-// is a pick). Every lane of the wave calls it (lane shuffles).
-__device__ inline void swiglu_pair_out(f4 gs, f4 us, float g0, float g1, int p, bool live, _Float16 *row) {
-    const int lg = (threadIdx.x % 64) / 16;
-    float mv[4], amax = 0.0f;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const float x = gs[r] * g0, uv = us[r] * g1;
-        mv[r] = __fmul_rn(__fdiv_rn(x, __fadd_rn(1.0f, expf(-x))), uv);
-        amax = fmaxf(amax, fabsf(mv[r]));
-    }
-    amax = fmaxf(amax, __shfl_xor(amax, 16, 64));
-    amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
-    const float sc = __fdiv_rn(amax, 127.0f), qi = amax > 0.0f ? __fdiv_rn(127.0f, amax) : 0.0f;
-    uint32_t hw[2], lw[2];   // this lane's 4 values (rows 4 lg .. 4 lg + 3 of the pair): hi, lo halves
-#pragma unroll
-    for (int r = 0; r < 4; r += 2) {
-        _Float16 h0, l0, h1, l1;
-        const int q0 = min(max(static_cast<int>(rintf(__fmul_rn(mv[r], qi))), -127), 127);
-        const int q1 = min(max(static_cast<int>(rintf(__fmul_rn(mv[r + 1], qi))), -127), 127);
-        const bool ex = g_act_exact != 0;   // (the exact path: the SwiGLU values themselves)
-        split_f16(ex ? mv[r] : __fmul_rn(static_cast<float>(q0), sc), h0, l0);
-        split_f16(ex ? mv[r + 1] : __fmul_rn(static_cast<float>(q1), sc), h1, l1);
-        hw[r / 2] = static_cast<uint32_t>(__builtin_bit_cast(uint16_t, h0)) |
-                    (static_cast<uint32_t>(__builtin_bit_cast(uint16_t, h1)) << 16);
-        lw[r / 2] = static_cast<uint32_t>(__builtin_bit_cast(uint16_t, l0)) |
-                    (static_cast<uint32_t>(__builtin_bit_cast(uint16_t, l1)) << 16);
-    }
-    // k-group 2 p + lg / 2 holds values 0..3 (lane lg even) and 4..7 (lane lg + 1) in the slot order
-    // (0 4 1 5 2 6 3 7): the even lane takes its partner's four and writes the group
-    uint32_t ph[2], pl[2];
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-        ph[k] = __shfl_xor(hw[k], 16, 64);
-        pl[k] = __shfl_xor(lw[k], 16, 64);
-    }
-    if ((lg & 1) == 0 && live) {
-        auto inter = [](uint32_t mine, uint32_t other) {   // (m0, o0), (m1, o1) as two words
-            return make_uint2((mine & 0xFFFFu) | (other << 16), (mine >> 16) | (other & 0xFFFF0000u));
-        };
-        const uint2 h01 = inter(hw[0], ph[0]), h23 = inter(hw[1], ph[1]);
-        const uint2 l01 = inter(lw[0], pl[0]), l23 = inter(lw[1], pl[1]);
-        const int gi = 2 * p + lg / 2;
-        uint4 *dst = reinterpret_cast<uint4 *>(row + static_cast<int64_t>(gi) * 16);
-        dst[0] = make_uint4(h01.x, h01.y, h23.x, h23.y);
-        dst[1] = make_uint4(l01.x, l01.y, l23.x, l23.y);
-    }
-}
-
 // SW (UP): the workgroup's tiles are matched gate / up pairs (gate tile p, up tile F / 16 + p: the tile loop takes
 // them in turns, tiles_per_wg even), and each flush of two pairs writes their SwiGLU's operands for down
 // (swiglu_pair_out) to sw_out [pick] instead of the products to out: no gate|up buffer, no SwiGLU launch.

@@ -266,7 +266,7 @@ __global__ __launch_bounds__(64 * WMAX) void gemv_q4_kernel(Q4 w, const _Float16
 #pragma unroll
         for (int r = 0; r < 4; ++r) old[r] = p[min(row0 + r, w.rows - 1)];   // (clamped: always a valid address)
     };
-    mfma_tiles<KW, NTT, kKeepParts, NT, (NT > 0 ? NT : 3), PACK>(
+    mfma_tiles<KW, NTT, kKeepParts, NT, (NT == 0 ? 3 : NT == 1 ? 2 : NT), PACK>(
         w.codes, w.scales, w.rows, static_cast<int>(w.cols / kSuperK), sc0, nt, M,
         [&](int j) { return act + j * act_stride; }, [](int64_t, int, float) {}, part_lds, tab, TileRun{t0}, prefetch,
         [&] { if (tc >= 0) trace(tc, 5); });
@@ -397,74 +397,34 @@ __global__ __launch_bounds__(256) void quantize_f16_kernel(const uint16_t *__res
     norm_quant_regs(v, cols, nullptr, 0.0f, act + static_cast<int64_t>(t) * act_stride, nullptr, red);
 }
 
-// The gate and up products with the SwiGLU and its quantization in one launch: a workgroup per 16-row tile pair
-// (gate tile p, up tile p), its waves splitting K as the skinny product does (the same sums, in the same order); the
-// 16 values m = silu(g) x u of a row and tile are one quantization block, so the down product's operands are the
-// workgroup's own (at most 8 rows: the rows' hi and lo halves in the MFMA's columns).
-template <int KW>
-__global__ __launch_bounds__(256) void ffn_up_kernel(Q4 gate, Q4 up, const _Float16 *__restrict__ act,
+// The gate and up products with the SwiGLU and its quantization in one launch, up to 32 rows: a workgroup per 16-row
+// tile pair (gate tile p, up tile p), its waves splitting K; the 16 values m = silu(g) x u of a row and tile are one
+// quantization block, so the down product's operands are the workgroup's own (swiglu_pair_out). Both tiles' loads are
+// in flight at once (a matrix pair as one call's two tiles): bound by the latency of that one round of loads, which
+// eight waves (half the K range each, three waves a SIMD at 384 workgroups) wait for together.
+// 2048 -> 6144, 5 rows: 10.9 us with the two products one after the other on four waves, 8.4 so.
+// (NP pairs a workgroup: at 17..32 rows its operands are several times its weights)
+template <int KW, int NTT, bool PACK, int NP>
+__global__ __launch_bounds__(512) void ffn_up_kernel(Q4 gate, Q4 up, const _Float16 *__restrict__ act,
                                                      int64_t act_stride, int M, _Float16 *__restrict__ act_m,
                                                      int64_t act_m_stride) {
     extern __shared__ f4 part_lds[];
     __shared__ uint2 tab[256];
-    const int p = blockIdx.x, W = blockDim.x / 64, lane = threadIdx.x % 64;
-    const int nsc = static_cast<int>(gate.cols / kSuperK);
-    auto rowp = [&](int j) { return act + static_cast<int64_t>(min(j, M - 1)) * act_stride; };
-    auto tile = [&](int) -> int64_t { return p; };
-    mfma_tiles<KW, 1, kKeepParts, 1, 2, true>(gate.codes, gate.scales, gate.rows, nsc, 0, 1, M, rowp,
-                                              [](int64_t, int, float) {}, part_lds, tab, tile);
-    mfma_tiles<KW, 1, kKeepParts, 1, 2, true>(up.codes, up.scales, up.rows, nsc, 0, 1, M, rowp,
-                                              [](int64_t, int, float) {}, part_lds + W * 64, tab, tile);
-    if (threadIdx.x >= 64) return;
-    // the waves' sums in wave order x global (the products' put), m = silu(g) x u (swiglu's arithmetic), the block's
-    // operands (quantize_activation); lane (j = lane % 16, lg = lane / 16): rows 4 lg .. 4 lg + 3 of the tile, row j
-    const int j = lane % 16, lg = lane / 16;
-    f4 gs = part_lds[lane], us = part_lds[W * 64 + lane];
-    for (int w2 = 1; w2 < W; ++w2) {
-        gs += part_lds[w2 * 64 + lane];
-        us += part_lds[(W + w2) * 64 + lane];
-    }
-    float mv[4], amax = 0.0f;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const float x = gs[r] * gate.global, uv = us[r] * up.global;
-        mv[r] = __fmul_rn(__fdiv_rn(x, __fadd_rn(1.0f, expf(-x))), uv);
-        amax = fmaxf(amax, fabsf(mv[r]));
-    }
-    amax = fmaxf(amax, __shfl_xor(amax, 16, 64));
-    amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
-    const float sc = __fdiv_rn(amax, 127.0f), qi = amax > 0.0f ? __fdiv_rn(127.0f, amax) : 0.0f;
-    uint32_t hw[2], lw[2];
-#pragma unroll
-    for (int r = 0; r < 4; r += 2) {
-        _Float16 h0, l0, h1, l1;
-        const int q0 = min(max(static_cast<int>(rintf(__fmul_rn(mv[r], qi))), -127), 127);
-        const int q1 = min(max(static_cast<int>(rintf(__fmul_rn(mv[r + 1], qi))), -127), 127);
-        const bool ex = g_act_exact != 0;   // (the exact path: the SwiGLU values themselves)
-        split_f16(ex ? mv[r] : __fmul_rn(static_cast<float>(q0), sc), h0, l0);
-        split_f16(ex ? mv[r + 1] : __fmul_rn(static_cast<float>(q1), sc), h1, l1);
-        hw[r / 2] = static_cast<uint32_t>(__builtin_bit_cast(uint16_t, h0)) |
-                    (static_cast<uint32_t>(__builtin_bit_cast(uint16_t, h1)) << 16);
-        lw[r / 2] = static_cast<uint32_t>(__builtin_bit_cast(uint16_t, l0)) |
-                    (static_cast<uint32_t>(__builtin_bit_cast(uint16_t, l1)) << 16);
-    }
-    // k-group 2 p + lg / 2 holds values 0..3 (lane lg even) and 4..7 (lane lg + 1) in the slot order
-    // (0 4 1 5 2 6 3 7): the even lane takes its partner's four and writes the group
-    uint32_t ph[2], pl[2];
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-        ph[k] = __shfl_xor(hw[k], 16, 64);
-        pl[k] = __shfl_xor(lw[k], 16, 64);
-    }
-    if ((lg & 1) == 0 && j < M) {
-        auto inter = [](uint32_t mine, uint32_t other) {
-            return make_uint2((mine & 0xFFFFu) | (other << 16), (mine >> 16) | (other & 0xFFFF0000u));
-        };
-        const uint2 h01 = inter(hw[0], ph[0]), h23 = inter(hw[1], ph[1]);
-        const uint2 l01 = inter(lw[0], pl[0]), l23 = inter(lw[1], pl[1]);
-        uint4 *dst = reinterpret_cast<uint4 *>(act_m + j * act_m_stride + static_cast<int64_t>(2 * p + lg / 2) * 16);
-        dst[0] = make_uint4(h01.x, h01.y, h23.x, h23.y);
-        dst[1] = make_uint4(l01.x, l01.y, l23.x, l23.y);
+    const int W = blockDim.x / 64, npair = static_cast<int>(gate.rows / kTileR);
+    const int p0 = static_cast<int>(blockIdx.x) * NP, np = min(NP, npair - p0);
+    mfma_tiles_of<KW, NTT, kKeepParts, 2 * NP, 2 * NP < 3 ? 2 * NP : 3, PACK>(
+        MatrixPair{gate.codes, gate.scales, up.codes, up.scales}, gate.rows, static_cast<int>(gate.cols / kSuperK), 0,
+        2 * np, M, [&](int j) { return act + static_cast<int64_t>(j) * act_stride; }, [](int64_t, int, float) {},
+        part_lds, tab, [&](int i) -> int64_t { return p0 + (i >> 1); });
+    for (int o = threadIdx.x; o < np * NTT * 64; o += blockDim.x) {   // a wave a pair and 16-column tile of rows
+        const int q = o / (NTT * 64), tt = (o / 64) % NTT, lane = o % 64, j = tt * 16 + lane % 16;
+        const f4 *gp = part_lds + (2 * q * W * NTT + tt) * 64 + lane, *up_ = gp + W * NTT * 64;
+        f4 gs = gp[0], us = up_[0];
+        for (int w2 = 1; w2 < W; ++w2) {   // the waves' sums in wave order
+            gs += gp[w2 * NTT * 64];
+            us += up_[w2 * NTT * 64];
+        }
+        swiglu_pair_out(gs, us, gate.global, up.global, p0 + q, j < M, act_m + j * act_m_stride);
     }
 }
 
@@ -475,21 +435,50 @@ int quantize_f16(const uint16_t *x, int M, int cols, _Float16 *act, int64_t act_
     return 0;
 }
 
-int ffn_up(const Q4 &gate, const Q4 &up, const _Float16 *act, int64_t act_stride, int M, _Float16 *act_m,
-           int64_t act_m_stride, hipStream_t st) {
+// K split over eight waves where it can be (half the decode chain of four), whole 16-row tiles
+static bool ffn_up_split(const Q4 &gate, int M, int &waves, int &kw) {
+    const int ntt = M <= 16 ? 1 : 2;
+    if (gate.rows % kTileR != 0 || !mfma_split(gate.cols, ntt, waves, kw)) return false;
+    if (waves <= 4 && kw == 16) kw = 8, waves *= 2;
+    return M <= 8 || kw <= 8;   // (unpacked: the hi and lo operands of 16 chunks do not fit a wave's registers twice)
+}
+bool ffn_up_fits(const Q4 &gate, const Q4 &up, int M) {
     int waves = 0, kw = 0;
-    GV_REQUIRE(M >= 1 && M <= 8 && gate.rows == up.rows && gate.cols == up.cols && gate.rows % kTileR == 0 &&
-                   mfma_split(gate.cols, 1, waves, kw) && waves <= 4,
-               "ffn_up: 1 <= M <= 8, gate and up alike, whole row tiles, K split over at most 4 waves");
-    const dim3 grid(static_cast<unsigned>(gate.rows / kTileR)), block(static_cast<unsigned>(64 * waves));
-    const size_t lds = static_cast<size_t>(2 * waves) * 1024;
-    if (kw == 16) hipLaunchKernelGGL(ffn_up_kernel<16>, grid, block, lds, st, gate, up, act, act_stride, M, act_m, act_m_stride);
-    else if (kw == 8) hipLaunchKernelGGL(ffn_up_kernel<8>, grid, block, lds, st, gate, up, act, act_stride, M, act_m, act_m_stride);
-    else hipLaunchKernelGGL(ffn_up_kernel<4>, grid, block, lds, st, gate, up, act, act_stride, M, act_m, act_m_stride);
+    return M >= 1 && M <= kMaxRows && gate.rows == up.rows && gate.cols == up.cols && ffn_up_split(gate, M, waves, kw);
+}
+
+template <int KW, int NTT, bool PACK, int NP>
+static int launch_ffn_up(const Q4 &gate, const Q4 &up, const _Float16 *act, int64_t act_stride, int M, int waves,
+                         _Float16 *act_m, int64_t act_m_stride, hipStream_t st) {
+    const int64_t npair = gate.rows / kTileR;
+    const size_t lds = static_cast<size_t>(2 * NP * waves * NTT) * 1024;   // at most 64 KB
+    hipLaunchKernelGGL((ffn_up_kernel<KW, NTT, PACK, NP>), dim3(static_cast<unsigned>((npair + NP - 1) / NP)),
+                       dim3(static_cast<unsigned>(64 * waves)), lds, st, gate, up, act, act_stride, M, act_m,
+                       act_m_stride);
     GV_CHECK_HIP(hipGetLastError());
     return 0;
 }
 
+int ffn_up(const Q4 &gate, const Q4 &up, const _Float16 *act, int64_t act_stride, int M, _Float16 *act_m,
+           int64_t act_m_stride, hipStream_t st) {
+    int waves = 0, kw = 0;
+    GV_REQUIRE(ffn_up_fits(gate, up, M) && ffn_up_split(gate, M, waves, kw),
+               "ffn_up: 1 <= M <= 32, gate and up alike, whole row tiles, K split over at most 8 waves");
+#define GV_FFN_UP(KW, NTT, PACK, NP) \
+    return launch_ffn_up<KW, NTT, PACK, NP>(gate, up, act, act_stride, M, waves, act_m, act_m_stride, st)
+    if (M <= 8) {
+        if (kw == 16) GV_FFN_UP(16, 1, true, 1);
+        if (kw == 8) GV_FFN_UP(8, 1, true, 1);
+        GV_FFN_UP(4, 1, true, 1);
+    }
+    if (M <= 16) {
+        if (kw == 8) GV_FFN_UP(8, 1, false, 1);
+        GV_FFN_UP(4, 1, false, 1);
+    }
+    if (kw == 8) GV_FFN_UP(8, 2, false, 2);
+    GV_FFN_UP(4, 2, false, 2);
+#undef GV_FFN_UP
+}
 
 int trace_set_q4(uint64_t *p) {
     GV_CHECK_HIP(hipMemcpyToSymbol(HIP_SYMBOL(g_trace), &p, sizeof p));
@@ -582,29 +571,52 @@ int gemv_q4(const Q4 &w, const _Float16 *act, int64_t act_stride, int M, const G
     GV_REQUIRE(w.cols % kSuperK == 0 && w.cols <= kMaxActCols, "gemv_q4: cols must be a multiple of 128, at most 16384");
     const int ntt = M <= 16 ? 1 : 2;
     const int nsc = static_cast<int>(w.cols / kSuperK);
-    if (ntt == 2 && nsc == 32) {   // 17..32 rows over K = 4096 (the tree's output projection), a few tiles: the rows in
-                                   // two groups of at most 16, each over the whole K in one range (the sums of an
-                                   // M <= 16 launch), both groups in one launch: twice the workgroups, each loading
-                                   // half the rows' operands
-        int waves, kw;
-        const int64_t ntiles = tiles_rows(w.rows);
-        if (mfma_split(32 * kSuperK, 1, waves, kw) && kw == 16 && waves == 8 && tiles_per_wg(ntiles, waves, 1) == 1) {
-            static int granted = 0;
-            if (lds_grant(reinterpret_cast<const void *>(&gemv_q4_kernel<16, 1, 8, false, 0, true>), 76 * 1024,
-                          granted) != 0)
-                return -1;
-            hipLaunchKernelGGL((gemv_q4_kernel<16, 1, 8, false, 0, true>), dim3(static_cast<unsigned>(ntiles), 2),
-                               dim3(64 * waves), static_cast<size_t>(waves) * 1024, st, w, act, act_stride, M, 0, 1,
-                               out);
+    const int64_t ntiles = tiles_rows(w.rows);
+    if (ntt == 2 && ntiles <= (nsc > 16 ? 256 : 128)) {
+        // 17..32 rows over few tiles (a tree's output projection, a dense MLP's down product): the rows in two groups of
+        // at most 16, both in one launch: twice the workgroups, each loading half the rows' operands (the sums of an
+        // M <= 16 launch). K in ranges of at most 4096; with the rows in one group the ranges are half that. Few: both
+        // groups' workgroups fit a round of the chip, or K needs the larger ranges. 2048 x 4096, 17 rows: 16.0 us in
+        // one group, 10.6 so; 2048 x 6144 in two ranges instead of three, 17 and 32 rows: the whole MLP 41 -> 30 and
+        // 51 -> 37 us; 4096 x 2048 at 17 rows the other way, 9.1 us against 10.6.
+        // (A matrix of more tiles than CUs streams many a workgroup and loses more by loading each twice: the 9216-row
+        // q|k|v product took the 40-layer step from 5.58 to 5.93 ms.)
+        GemvOut o = out;
+        for (int sc0 = 0; sc0 < nsc;) {
+            int n = std::min(nsc - sc0, 32), waves, kw;
+            while (n > 1 && !mfma_split(static_cast<int64_t>(n) * kSuperK, 1, waves, kw)) --n;
+            GV_REQUIRE(sc0 % 4 == 0 && mfma_split(static_cast<int64_t>(n) * kSuperK, 1, waves, kw),
+                       "gemv_q4: a K range must start on a quad of super-chunks");
+            if (kw == 16 && waves <= 4) kw = 8, waves *= 2;   // (half the decode chain, as gemv_range)
+            const dim3 grid(static_cast<unsigned>(ntiles), 2), block(static_cast<unsigned>(64 * waves));
+            const size_t lds = static_cast<size_t>(waves) * 1024;
+            if (kw == 16)
+                hipLaunchKernelGGL((gemv_q4_kernel<16, 1, 8, false, 0, true>), grid, block, lds, st, w, act, act_stride, M, sc0, 1, o);
+            else if (kw == 8)
+                hipLaunchKernelGGL((gemv_q4_kernel<8, 1, 8, false, 0, true>), grid, block, lds, st, w, act, act_stride, M, sc0, 1, o);
+            else
+                hipLaunchKernelGGL((gemv_q4_kernel<4, 1, 8, false, 0, true>), grid, block, lds, st, w, act, act_stride, M, sc0, 1, o);
             GV_CHECK_HIP(hipGetLastError());
-            return 0;
+            o.accumulate = 1;
+            sc0 += n;
         }
+        return 0;
+    }
+    if (M <= 8 && nsc > 32 && nsc <= 48 && nsc % 4 == 0 && ntiles <= 256) {
+        // K of 4096 .. 6144 over at most a tile a CU (a dense MLP's down product): one launch of up to twelve waves,
+        // 512 values each, instead of two K ranges one after the other - with a tile a workgroup a launch is one
+        // round of loads, so the second range's launch costs as much as the first's. More tiles (each CU streaming
+        // many) or wider K (the waves' operands no longer fit their registers): the ranges below.
+        const int waves = nsc / 4;
+        hipLaunchKernelGGL((gemv_q4_kernel<16, 1, 12, true, 1>), dim3(static_cast<unsigned>(ntiles)),
+                           dim3(64 * waves), static_cast<size_t>(waves) * 1024, st, w, act, act_stride, M, 0, 1, out);
+        GV_CHECK_HIP(hipGetLastError());
+        return 0;
     }
     // K ranges whose activations fit the waves' registers: one launch up to 4096 (2048 for 17..32 rows) values,
     // later ranges adding to the first's sums
     if (ntt == 2 && nsc == 32) {   // two ranges of 2048 in one launch (kept parts, up to two tiles a workgroup)
         int waves, kw;
-        const int64_t ntiles = tiles_rows(w.rows);
         if (mfma_split(16 * kSuperK, 2, waves, kw) && kw == 8 && waves == 8 && tiles_per_wg(ntiles, waves, 2) <= 2) {
             const int64_t per = tiles_per_wg(ntiles, waves, 2), wg = (ntiles + per - 1) / per;
             const size_t lds = static_cast<size_t>(2 * per) * waves * 2 * 1024;
