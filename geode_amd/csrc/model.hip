@@ -2379,6 +2379,9 @@ void gv_model_free(gv_model *g) {
     mtp_release(g->m);
     for (void *p : g->m.allocs) (void)hipFree(p);
     for (void *p : g->m.pf.allocs) (void)hipFree(p);
+    if (g->m.pf.stage) (void)hipHostFree(g->m.pf.stage);
+    for (hipEvent_t e : g->m.pf.stage_ev)
+        if (e) (void)hipEventDestroy(e);
     if (g->m.trace) {   // the kernels stop stamping before the buffer goes
         uint64_t *none = nullptr;
         (void)hipMemcpyToSymbol(HIP_SYMBOL(g_trace), &none, sizeof none);
@@ -2912,6 +2915,85 @@ int moe_block(Model &m, int layer, int M, bool given, hipStream_t st) {
     m.moe_only = false;
     return rc;
 }
+
+// ---------------------------------------------------------------- the MoE block's rows between host and device
+// The caller's rows are ordinary (pageable) memory, which the runtime copies at half the link's rate and, for rows of
+// another stride, one by one (512 rows of router logits: 4.7 ms). Here they go through pinned slots used in turn, the
+// host's copy of one slot beside the link's copies of the others. 512 rows, the whole call: 5.45 ms, 0.55 so (slots of
+// 1 or 2 MB; 0.64 with 512 KB and 0.86 with 256 KB, a copy's fixed ~10 us; 0.65 with 4 MB, too few to overlap).
+int stage_open(Model &m) {
+    Prefill &pf = m.pf;
+    if (!pf.stage) {
+        void *p = nullptr;
+        GV_CHECK_HIP(hipHostMalloc(&p, kStageSlots * kStageSlot, hipHostMallocDefault));
+        pf.stage = static_cast<char *>(p);
+    }
+    for (hipEvent_t &e : pf.stage_ev)
+        if (!e) GV_CHECK_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    return 0;
+}
+
+// `rows` rows of src_row bytes to rows of dst_row bytes on the device (the rest of a wider one: zeros)
+int stage_rows_in(Model &m, void *dst, const void *src, int64_t rows, size_t src_row, size_t dst_row, hipStream_t st) {
+    Prefill &pf = m.pf;
+    const bool plain = src_row == dst_row;
+    const size_t bytes = static_cast<size_t>(rows) * dst_row, step = plain ? kStageSlot : kStageSlot / dst_row * dst_row;
+    GV_REQUIRE(step > 0, "gv_model_moe: a row wider than a staging slot");
+    for (size_t o = 0; o < bytes; o += step) {
+        const size_t n = std::min(step, bytes - o);
+        const int s = pf.stage_next++ % kStageSlots;
+        char *slot = pf.stage + static_cast<size_t>(s) * kStageSlot;
+        GV_CHECK_HIP(hipEventSynchronize(pf.stage_ev[s]));   // (its last copy done: at once for an event never recorded)
+        if (plain) {
+            std::memcpy(slot, static_cast<const char *>(src) + o, n);
+        } else {
+            const char *from = static_cast<const char *>(src) + o / dst_row * src_row;
+            for (size_t d = 0; d < n; d += dst_row, from += src_row) {
+                std::memcpy(slot + d, from, src_row);
+                std::memset(slot + d + src_row, 0, dst_row - src_row);
+            }
+        }
+        GV_CHECK_HIP(hipMemcpyAsync(static_cast<char *>(dst) + o, slot, n, hipMemcpyHostToDevice, st));
+        GV_CHECK_HIP(hipEventRecord(pf.stage_ev[s], st));
+    }
+    return 0;
+}
+
+// Device pieces to the caller's memory, in order; returns once all of it is there (everything enqueued before, too)
+struct StagePiece {
+    void *dst;
+    const void *src;
+    size_t bytes;
+};
+int stage_out(Model &m, const StagePiece *piece, int pieces, hipStream_t st) {
+    Prefill &pf = m.pf;
+    struct Flight {
+        char *dst;
+        size_t n;
+        int slot;
+    } fl[kStageSlots];
+    int head = 0, tail = 0;   // flights [head, tail)
+    auto land = [&]() -> int {
+        const Flight &f = fl[head++ % kStageSlots];
+        GV_CHECK_HIP(hipEventSynchronize(pf.stage_ev[f.slot]));
+        std::memcpy(f.dst, pf.stage + static_cast<size_t>(f.slot) * kStageSlot, f.n);
+        return 0;
+    };
+    for (int i = 0; i < pieces; ++i)
+        for (size_t o = 0; o < piece[i].bytes; o += kStageSlot) {
+            if (tail - head == kStageSlots && land() != 0) return -1;
+            // (a slot still read by a copy in: the stream does that copy first)
+            const int s = pf.stage_next++ % kStageSlots;
+            const size_t n = std::min(kStageSlot, piece[i].bytes - o);
+            GV_CHECK_HIP(hipMemcpyAsync(pf.stage + static_cast<size_t>(s) * kStageSlot,
+                                        static_cast<const char *>(piece[i].src) + o, n, hipMemcpyDeviceToHost, st));
+            GV_CHECK_HIP(hipEventRecord(pf.stage_ev[s], st));
+            fl[tail++ % kStageSlots] = Flight{static_cast<char *>(piece[i].dst) + o, n, s};
+        }
+    while (head < tail)
+        if (land() != 0) return -1;
+    return 0;
+}
 }  // namespace gv
 
 extern "C" {
@@ -2934,26 +3016,28 @@ int gv_model_moe(gv_model *g, int layer, const float *h, int M, const float *rou
     std::memset(&sp, 0, sizeof sp);
     sp.pos = m.pos;
     sp.M = std::min(M, c.max_rows);
-    GV_CHECK_HIP(hipMemcpyAsync(m.sp, &sp, sizeof sp, hipMemcpyHostToDevice, st));
-    GV_CHECK_HIP(hipMemcpyAsync(pf.h, h, static_cast<size_t>(M) * H * 4, hipMemcpyHostToDevice, st));
-    if (router_logits)
-        GV_CHECK_HIP(hipMemcpy2DAsync(pf.logits, static_cast<size_t>(m.E1) * 4, router_logits,
-                                      static_cast<size_t>(E) * 4, static_cast<size_t>(E) * 4, M,
-                                      hipMemcpyHostToDevice, st));
+    if (stage_open(m) != 0) return -1;
+    // (the prefill path takes its row count as a kernel argument, the verify step's kernels from the step parameters)
+    if (M <= c.max_rows && stage_rows_in(m, m.sp, &sp, 1, sizeof sp, sizeof sp, st) != 0) return -1;
+    if (router_logits && stage_rows_in(m, pf.logits, router_logits, M, static_cast<size_t>(E) * 4,
+                                       static_cast<size_t>(m.E1) * 4, st) != 0)
+        return -1;
+    if (stage_rows_in(m, pf.h, h, 1, static_cast<size_t>(M) * H * 4, static_cast<size_t>(M) * H * 4, st) != 0) return -1;
     GV_REQUIRE(moe_block(m, layer, M, router_logits != nullptr, st) == 0,
                std::string("gv_model_moe: ") + last_error());
     pf.M = M;
     pf.given = router_logits != nullptr;
     pf.layer = layer;
     const bool big = M > c.max_rows;
-    GV_CHECK_HIP(hipMemcpyAsync(out, big ? pf.out : m.x, static_cast<size_t>(M) * H * 4, hipMemcpyDeviceToHost, st));
-    if (ids)
-        GV_CHECK_HIP(hipMemcpyAsync(ids, big ? pf.ids : m.route_ids + static_cast<int64_t>(layer) * c.max_rows * K,
-                                    static_cast<size_t>(M) * K * 4, hipMemcpyDeviceToHost, st));
-    if (weights)
-        GV_CHECK_HIP(hipMemcpyAsync(weights, big ? pf.w : m.route[layer].weight, static_cast<size_t>(M) * K * 4,
-                                    hipMemcpyDeviceToHost, st));
-    if (check_wait_flag(m, st) != 0) return -1;   // (synchronizes the stream)
+    const size_t picks = static_cast<size_t>(M) * K * 4;
+    int flag = 0;
+    const StagePiece out_pieces[] = {
+        {ids, big ? pf.ids : m.route_ids + static_cast<int64_t>(layer) * c.max_rows * K, ids ? picks : 0},
+        {weights, big ? pf.w : m.route[layer].weight, weights ? picks : 0},
+        {&flag, m.err, 4},
+        {out, big ? pf.out : m.x, static_cast<size_t>(M) * H * 4}};
+    if (stage_out(m, out_pieces, 4, st) != 0) return -1;
+    GV_REQUIRE(flag == 0, "gv_model_moe: a fused launch's wait for its producers ran out (the results are invalid)");
     m.last_n = 0;   // the step's state is this block's, not a verify's
     return 0;
 }

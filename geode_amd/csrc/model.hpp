@@ -97,7 +97,14 @@ struct Prefill {
     _Float16 *act = nullptr, *act_m = nullptr;
     int max_slots = 0, max_picks = 0;
     std::vector<void *> allocs;
+    // gv_model_moe's rows on their way between the caller's memory and the device: pinned slots used in turn, an event
+    // a slot (allocated on the first call, given back with the model)
+    char *stage = nullptr;
+    hipEvent_t stage_ev[8] = {};
+    int stage_next = 0;
 };
+constexpr int kStageSlots = 8;
+constexpr size_t kStageSlot = size_t{1} << 20;
 
 struct Model {
     gv_model_config c{};
