@@ -320,19 +320,25 @@ enum TilesMode { kSplitK = 0, kKeepParts = 1, kWaveTiles = 2 };
 // part: LDS of max(nt, NT) * W * NTT KB for the waves' partial sums (kSplitK, kKeepParts: part[((i W + w) NTT + tt)
 // 64 + lane], left there after a workgroup barrier in kKeepParts); FLUSH > 0 (kSplitK, runtime loop): the sums of
 // every FLUSH tiles are put as soon as those tiles are done, so part holds FLUSH * W * NTT KB whatever nt is (the
-// activations stay in registers over many tiles); tab: LDS for fill_e4m3_table, filled here. hook()
+// activations stay in registers over many tiles); BUFS 2 (with a flush of the call's own): two such halves of part in
+// turn, so a wave that has put its share goes on while others still read it (one barrier a flush: a half is written
+// again only after the next flush's barrier, which its readers have passed); PACK 2 (NTT 2, M <= 24): the second
+// column tile packed, three MFMAs a word instead of four; tab: LDS for fill_e4m3_table, filled here. hook()
 // runs after the first tiles' loads are issued and before the activations are loaded (a wait for them); ready() once
 // the activations and the first tiles are in registers. Every thread of the workgroup calls this.
-template <int KW, int NTT, int MODE, int NT = 0, int DEPTH = 3, bool PACK = false, int FLUSH = 0, typename RowFn,
-          typename PutFn, typename MapFn = TileRun, typename HookFn = NoHook, typename ReadyFn = NoHook,
-          typename FlushFn = NoFlush, typename MatFn = OneMatrix>
+template <int KW, int NTT, int MODE, int NT = 0, int DEPTH = 3, int PACK = 0, int FLUSH = 0, int BUFS = 1,
+          typename RowFn, typename PutFn, typename MapFn = TileRun, typename HookFn = NoHook,
+          typename ReadyFn = NoHook, typename FlushFn = NoFlush, typename MatFn = OneMatrix>
 __device__ inline void mfma_tiles_of(const MatFn mat, int64_t rows, int nsc, int sc0, int nt, int M, RowFn rowp,
                                      PutFn put, f4 *part, uint2 *tab, MapFn tmap, HookFn hook = HookFn{},
                                      ReadyFn ready = ReadyFn{}, FlushFn flush = FlushFn{}) {
     static_assert(DEPTH >= 2 && (NT > 0 || DEPTH >= 3), "the runtime loop is a ring of at least three");
-    static_assert(!PACK || NTT == 1, "packed hi | lo columns take one 16-row tile of at most 8 rows");
+    static_assert(PACK <= 1 || NTT == 2, "packed after a whole tile: two tiles, at most 24 rows");
+    static_assert(PACK != 1 || NTT == 1, "packed hi | lo columns take one 16-row tile of at most 8 rows");
+    static_assert(BUFS == 1 || FLUSH > 0, "turns are of the flushed tiles");
     static_assert(FLUSH == 0 || (MODE == kSplitK && NT == 0), "the flushed split-K runs the runtime tile loop");
-    constexpr int NB = PACK ? 1 : 2;   // operand arrays: hi | lo packed, or hi and lo
+    constexpr int NB = PACK == 1 ? 1 : 2;   // operand arrays: hi | lo packed, or hi and lo
+    constexpr auto packed = [](int tt) { return PACK == 1 || (PACK == 2 && tt == 1); };   // (column tile tt)
     const int W = MODE == kWaveTiles ? 1 : static_cast<int>(blockDim.x / 64);
     const int w = MODE == kWaveTiles ? 0 : static_cast<int>(threadIdx.x / 64);
     const int l = threadIdx.x % 64, lq = l % 16, lg = l / 16;
@@ -380,12 +386,12 @@ __device__ inline void mfma_tiles_of(const MatFn mat, int64_t rows, int nsc, int
     h8 b[NB][KW][NTT];
 #pragma unroll
     for (int tt = 0; tt < NTT; ++tt) {
-        const int j = PACK ? lq % 8 : tt * 16 + lq;
+        const int j = tt * 16 + (packed(tt) ? lq % 8 : lq);
         const _Float16 *row = j < M ? rowp(j) : reinterpret_cast<const _Float16 *>(g_zero_act16);
 #pragma unroll
         for (int c = 0; c < KW; ++c) {
             const int64_t g = (static_cast<int64_t>(sc0) * 4 + w * KW + c) * 4 + lg;
-            if (PACK) {
+            if (packed(tt)) {
                 b[0][c][tt] = *reinterpret_cast<const h8 *>(row + g * 16 + (lq >= 8 ? 8 : 0));
             } else {
                 b[0][c][tt] = *reinterpret_cast<const h8 *>(row + g * 16);
@@ -425,14 +431,14 @@ __device__ inline void mfma_tiles_of(const MatFn mat, int64_t rows, int nsc, int
 #pragma unroll
                     for (int tt = 0; tt < NTT; ++tt)
 #pragma unroll
-                        for (int h = 0; h < NB; ++h)
+                        for (int h = 0; h < (packed(tt) ? 1 : NB); ++h)
                             acc[h][tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b[h][c][tt], acc[h][tt], 0, 0, 0);
                 }
             }
         }
 #pragma unroll
         for (int tt = 0; tt < NTT; ++tt) {
-            if (PACK) {   // column j < 8: hi sum + the lo sum from column j + 8 (lane l ^ 8)
+            if (packed(tt)) {   // column j < 8: hi sum + the lo sum from column j + 8 (lane l ^ 8)
                 f4 lo;
 #pragma unroll
                 for (int r = 0; r < 4; ++r) lo[r] = xor8(acc[0][tt][r]);
@@ -444,7 +450,7 @@ __device__ inline void mfma_tiles_of(const MatFn mat, int64_t rows, int nsc, int
         f4 (&res)[NTT] = acc[0];
         if (MODE != kWaveTiles) {
 #pragma unroll
-            for (int tt = 0; tt < NTT; ++tt) part[(((FLUSH ? i % FLUSH : i) * W + w) * NTT + tt) * 64 + l] = res[tt];
+            for (int tt = 0; tt < NTT; ++tt) part[(((FLUSH ? i % (BUFS * FLUSH) : i) * W + w) * NTT + tt) * 64 + l] = res[tt];
         } else if (i < nt) {
             const int64_t T = tmap(i);
 #pragma unroll
@@ -463,8 +469,8 @@ __device__ inline void mfma_tiles_of(const MatFn mat, int64_t rows, int nsc, int
     auto split_k_out = [&](int i0, int i1) {
         __syncthreads();
         if constexpr (FlushFn::active) {
-            flush(i0, i1, part, W);
-            if (FLUSH) __syncthreads();
+            flush(i0, i1, part + (FLUSH ? i0 % (BUFS * FLUSH) : 0) * W * NTT * 64, W);
+            if (FLUSH && BUFS == 1) __syncthreads();
             return;
         }
         for (int o = threadIdx.x; o < (i1 - i0) * NTT * 64; o += blockDim.x) {
@@ -517,14 +523,14 @@ __device__ inline void mfma_tiles_of(const MatFn mat, int64_t rows, int nsc, int
 }
 
 // mfma_tiles_of over one matrix
-template <int KW, int NTT, int MODE, int NT = 0, int DEPTH = 3, bool PACK = false, int FLUSH = 0, typename RowFn,
-          typename PutFn, typename MapFn = TileRun, typename HookFn = NoHook, typename ReadyFn = NoHook,
-          typename FlushFn = NoFlush>
+template <int KW, int NTT, int MODE, int NT = 0, int DEPTH = 3, int PACK = 0, int FLUSH = 0, int BUFS = 1,
+          typename RowFn, typename PutFn, typename MapFn = TileRun, typename HookFn = NoHook,
+          typename ReadyFn = NoHook, typename FlushFn = NoFlush>
 __device__ inline void mfma_tiles(const uint8_t *__restrict__ codes, const uint8_t *__restrict__ scales, int64_t rows,
                                   int nsc, int sc0, int nt, int M, RowFn rowp, PutFn put, f4 *part, uint2 *tab,
                                   MapFn tmap, HookFn hook = HookFn{}, ReadyFn ready = ReadyFn{},
                                   FlushFn flush = FlushFn{}) {
-    mfma_tiles_of<KW, NTT, MODE, NT, DEPTH, PACK, FLUSH>(OneMatrix{codes, scales}, rows, nsc, sc0, nt, M, rowp, put,
+    mfma_tiles_of<KW, NTT, MODE, NT, DEPTH, PACK, FLUSH, BUFS>(OneMatrix{codes, scales}, rows, nsc, sc0, nt, M, rowp, put,
                                                          part, tab, tmap, hook, ready, flush);
 }
 

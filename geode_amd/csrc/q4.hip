@@ -355,22 +355,47 @@ __global__ __launch_bounds__(64 * WMAX) void gemv_q4_2pass_kernel(Q4 w, const _F
 // The skinny product over many row tiles a workgroup at 17..32 rows (two 16-column tiles: a K range's activations
 // take half the registers, so the kept-parts form above holds only 4 tiles' partial sums and each workgroup reloads
 // the rows' activations every 4 tiles): the waves' sums put every kGemvFlush tiles (mfma_tiles FLUSH), the same
-// sums in the same order as gemv_q4_kernel, so a workgroup takes ~19 tiles with one load of the activations.
-constexpr int kGemvFlush = 4;
-template <int KW, int WMAX>
+// sums in the same order as gemv_q4_kernel. A round of the chip's workgroups takes every tile, a stride of the grid
+// apart (all of them read adjacent tiles at a time, at most one tile more than the others), so the activations are
+// loaded once a CU. The waves of the CU's one workgroup (their operands take 8 x 180 registers a lane) wait for one
+// another at a flush only: two halves of the partial sums in turn, one barrier each. PACK 2: at most 24 rows, the
+// second column tile's hi and lo halves in one MFMA.
+// The 151,936 x 2048 head at 17 rows, with its norm's launch: 62.9 us with four tiles a flush in one buffer over two
+// rounds of workgroups; one store a lane 4 rows, packed, two buffers 56.2; one round of workgroups 49.2; two tiles a
+// flush 47.7 (one: 52.5); strided tiles 46.6 (its weights and logits at a copy's rate: 36). Sixteen waves of half the
+// K range each: 58.
+constexpr int kGemvFlush = 2;
+template <int KW, int WMAX, int PACK>
 __global__ __launch_bounds__(64 * WMAX) void gemv_q4_flush_kernel(Q4 w, const _Float16 *__restrict__ act,
-                                                                  int64_t act_stride, int M, int sc0, int tiles_per_wg,
-                                                                  GemvOut out) {
+                                                                  int64_t act_stride, int M, int sc0, GemvOut out) {
     extern __shared__ f4 part_lds[];
     __shared__ uint2 tab[256];
-    const int64_t ntiles = tiles_rows(w.rows);
-    const int64_t t0 = static_cast<int64_t>(blockIdx.x) * tiles_per_wg;
-    if (t0 >= ntiles) return;
-    const int nt = static_cast<int>(std::min<int64_t>(tiles_per_wg, ntiles - t0));
-    mfma_tiles<KW, 2, kSplitK, 0, 3, false, kGemvFlush>(
+    const int ntiles = static_cast<int>(tiles_rows(w.rows));
+    const int wg = static_cast<int>(blockIdx.x), nwg = static_cast<int>(gridDim.x);   // (at most ntiles workgroups)
+    const int nt = (ntiles - wg + nwg - 1) / nwg;
+    // a lane's four rows of a column in one store: one segment, whole row tiles, 16-byte rows of y
+    const bool whole = !out.accumulate && out.nseg == 1 && w.rows % kTileR == 0 &&
+                       (reinterpret_cast<uintptr_t>(out.y) | static_cast<uintptr_t>(out.ldy) * 4) % 16 == 0;
+    auto tile_of = [&](int i) -> int64_t { return wg + static_cast<int64_t>(i) * nwg; };
+    mfma_tiles<KW, 2, kSplitK, 0, 4, PACK, kGemvFlush, 2>(
         w.codes, w.scales, w.rows, static_cast<int>(w.cols / kSuperK), sc0, nt, M,
-        [&](int j) { return act + j * act_stride; }, [&](int64_t row, int j, float v) { out.put(row, j, v); },
-        part_lds, tab, TileRun{t0});
+        [&](int j) { return act + j * act_stride; }, [](int64_t, int, float) {}, part_lds, tab, tile_of, NoHook{},
+        NoHook{}, flush_with([&](int i0, int i1, const f4 *part, int W) {   // a tile and column tile a lane: wave order
+            for (int o = threadIdx.x; o < (i1 - i0) * 128; o += blockDim.x) {
+                const int i = o / 128, tt = (o / 64) % 2, ll = o % 64, j = tt * 16 + ll % 16;
+                if (j >= M) continue;
+                f4 sum = part[(i * W * 2 + tt) * 64 + ll];
+                for (int w2 = 1; w2 < W; ++w2) sum += part[((i * W + w2) * 2 + tt) * 64 + ll];
+                const int64_t row0 = tile_of(i0 + i) * kTileR + 4 * (ll / 16);
+                if (whole) {
+                    *reinterpret_cast<f4 *>(out.y + j * out.ldy + row0) = sum * out.seg_global[0];
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        if (row0 + r < w.rows) out.put(row0 + r, j, sum[r]);
+                }
+            }
+        }));
 }
 
 GV_ACT_MODE_SETTER(act_mode_set_q4)
@@ -508,17 +533,17 @@ static int launch_gemv(const Q4 &w, const _Float16 *act, int64_t act_stride, int
     const int64_t per = tiles_per_wg(ntiles, waves, NTT);
     if constexpr (NTT == 2 && !PACK) {
         // a matrix whose tiles outnumber 4 a workgroup of the chip's resident ones (the head at a tree's 17 rows):
-        // the flushed form, ~2 workgroups a CU's worth of tiles each
+        // the flushed form, the resident workgroups over all the tiles
         const int64_t resident = 256 * std::max(1, 8 / waves);
         if (ntiles > per * resident) {
-            const int64_t pf = std::max<int64_t>(kGemvFlush, (ntiles + 2 * resident - 1) / (2 * resident));
-            const int64_t wgf = (ntiles + pf - 1) / pf;
-            const size_t ldsf = static_cast<size_t>(kGemvFlush) * waves * NTT * 1024;
-            static int granted_f = 0;
-            if (lds_grant(reinterpret_cast<const void *>(&gemv_q4_flush_kernel<KW, WMAX>), 76 * 1024, granted_f) != 0)
-                return -1;
-            hipLaunchKernelGGL((gemv_q4_flush_kernel<KW, WMAX>), dim3(static_cast<unsigned>(wgf)), dim3(64 * waves), ldsf,
-                               st, w, act, act_stride, M, sc0, static_cast<int>(pf), out);
+            const dim3 grid(static_cast<unsigned>(std::min(ntiles, resident))), block(static_cast<unsigned>(64 * waves));
+            const size_t lds = static_cast<size_t>(2 * kGemvFlush) * waves * NTT * 1024;   // at most 64 KB
+            if (M <= 24)
+                hipLaunchKernelGGL((gemv_q4_flush_kernel<KW, WMAX, 2>), grid, block, lds, st, w, act, act_stride, M, sc0,
+                                   out);
+            else
+                hipLaunchKernelGGL((gemv_q4_flush_kernel<KW, WMAX, 0>), grid, block, lds, st, w, act, act_stride, M, sc0,
+                                   out);
             return 0;
         }
     }
