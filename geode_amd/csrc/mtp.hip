@@ -35,13 +35,15 @@ struct PickArea {
     int count;   // finished workgroups of the running pick launch (zero between launches)
     int draft;
     float prob;
+    int err;     // the fused launches' error flag after the pass (read with the result in one copy)
 };
 
 // ---------------------------------------------------------------- kernels
 // fc's operands of row t (forward_mtp, model.cpp:4992-5008): the embedding of tokens[t] (dequant_row) normalized with
 // 1 + pre_e in values [0, H), the hidden row hrow[t] of hbuf normalized with 1 + pre_h in [H, 2 H), each as the int8
 // path's 16-value blocks (quantize_activation on the 2 H row: its blocks lie within one half, H being a multiple of
-// 16). A workgroup a row.
+// 16). A workgroup a (row, half): the two halves' norms side by side (5 rows of 2048: 7.3 us one after the other, 5.4
+// so).
 __global__ __launch_bounds__(256) void mtp_in_kernel(Q4 emb, const StepParams *__restrict__ sp,
                                                      const float *__restrict__ hbuf, const float *__restrict__ pre_e,
                                                      const float *__restrict__ pre_h, float eps,
@@ -50,10 +52,13 @@ __global__ __launch_bounds__(256) void mtp_in_kernel(Q4 emb, const StepParams *_
     const int t = blockIdx.x;
     if (t >= sp->M) return;
     const int H = static_cast<int>(emb.cols);
-    float v[4][8];
-    dequant_row_regs(emb, sp->tokens[t], v, nullptr);
     _Float16 *ar = act + static_cast<int64_t>(t) * act_stride;
-    norm_quant_regs(v, H, pre_e, eps, ar, nullptr, red);
+    if (blockIdx.y == 0) {   // (uniform)
+        float v[4][8];
+        dequant_row_regs(emb, sp->tokens[t], v, nullptr);
+        norm_quant_regs(v, H, pre_e, eps, ar, nullptr, red);
+        return;
+    }
     norm_quant_row(hbuf + static_cast<int64_t>(sp->hrow[t]) * H, H, pre_h, eps, ar + act_halves(H), nullptr, red);
 }
 
@@ -71,7 +76,8 @@ __device__ inline void wave_best(float &v, int &i) {
 __device__ inline int pick_chunk(int rows) { return (rows + kPickWgs - 1) / kPickWgs; }
 
 // The maximum: per chunk its largest logit and first index (sc1 stores), then the last workgroup to finish takes the
-// chunks in order (a later chunk only with a larger value: the first maximum) into maxv / best.
+// chunks, a lane each (the largest value, of equal ones the lowest index: the first maximum), into maxv / best. Bound by
+// the chain launch, chunk, hand-off, chunks: 32,000 rows 10.9 us with one thread over the chunks, 4.8 so.
 __global__ __launch_bounds__(kPickThreads) void pick_max_kernel(const float *__restrict__ lg, int rows, PickArea *pa) {
     __shared__ float sv[kPickThreads / 64];
     __shared__ int si[kPickThreads / 64];
@@ -92,24 +98,24 @@ __global__ __launch_bounds__(kPickThreads) void pick_max_kernel(const float *__r
         last = __hip_atomic_fetch_add(&pa->count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == kPickWgs - 1;
     }
     __syncthreads();
-    if (!last || threadIdx.x != 0) return;
-    float mv = -INFINITY;
-    int mi = INT32_MAX;
-    for (int c = 0; c < kPickWgs; ++c) {
-        const float cv = xldf(pa->chunk_max, c);
-        const int ci = __builtin_bit_cast(int, xldf(reinterpret_cast<const float *>(pa->chunk_idx), c));
-        if (cv > mv) mv = cv, mi = ci;   // (an empty chunk: -inf, never taken)
-    }
+    if (!last || threadIdx.x >= 64) return;
+    static_assert(kPickWgs == 64, "a chunk a lane");
+    float mv = xldf(pa->chunk_max, threadIdx.x);
+    int mi = __builtin_bit_cast(int, xldf(reinterpret_cast<const float *>(pa->chunk_idx), threadIdx.x));
+    wave_best(mv, mi);
+    if (threadIdx.x != 0) return;
+    if (mv == -INFINITY) mi = INT32_MAX;   // (no logit above -inf: none taken)
     pa->maxv = mv;
-    pa->best = mi >= 0 && mi < rows ? mi : 0;   // (no maximum only when every logit is NaN)
+    pa->best = mi >= 0 && mi < rows ? mi : 0;   // (no maximum only when every logit is NaN or -inf)
     __hip_atomic_store(&pa->count, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // The probability: per chunk sum exp(double(l - max)) (the difference in fp32 as the reference's, softmax_at), then the
-// last workgroup adds the chunks' sums in order: prob = 1 / sum, draft = the best index (through ids when a draft
-// vocabulary is set).
+// last workgroup adds the chunks' sums in order (read a lane each): prob = 1 / sum, draft = the best index (through ids
+// when a draft vocabulary is set). 32,000 rows: 6.2 us with one thread reading the sums, 4.9 so.
 __global__ __launch_bounds__(kPickThreads) void pick_sum_kernel(const float *__restrict__ lg, int rows,
-                                                                const int32_t *__restrict__ ids, PickArea *pa) {
+                                                                const int32_t *__restrict__ ids,
+                                                                const int *__restrict__ err, PickArea *pa) {
     __shared__ double sd[kPickThreads / 64];
     __shared__ int last;
     const int b = blockIdx.x, chunk = pick_chunk(rows);
@@ -131,14 +137,19 @@ __global__ __launch_bounds__(kPickThreads) void pick_sum_kernel(const float *__r
         last = __hip_atomic_fetch_add(&pa->count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == kPickWgs - 1;
     }
     __syncthreads();
-    if (!last || threadIdx.x != 0) return;
+    if (!last || threadIdx.x >= 64) return;
+    const int lo32 = __builtin_bit_cast(int, xldf(pa->chunk_sum, 2 * static_cast<int>(threadIdx.x)));
+    const int hi32 = __builtin_bit_cast(int, xldf(pa->chunk_sum, 2 * static_cast<int>(threadIdx.x) + 1));
     double tot = 0.0;
+#pragma unroll
     for (int c = 0; c < kPickWgs; ++c) {
-        const uint64_t lo32 = __builtin_bit_cast(uint32_t, xldf(pa->chunk_sum, 2 * c));
-        const uint64_t hi32 = __builtin_bit_cast(uint32_t, xldf(pa->chunk_sum, 2 * c + 1));
-        tot += __builtin_bit_cast(double, lo32 | (hi32 << 32));
+        const uint64_t l = static_cast<uint32_t>(__builtin_amdgcn_readlane(lo32, c));
+        const uint64_t h = static_cast<uint32_t>(__builtin_amdgcn_readlane(hi32, c));
+        tot += __builtin_bit_cast(double, l | (h << 32));
     }
+    if (threadIdx.x != 0) return;
     pa->prob = static_cast<float>(1.0 / tot);
+    pa->err = *err;   // (every earlier launch of the pass is done)
     pa->draft = ids ? ids[pa->best] : pa->best;
     __hip_atomic_store(&pa->count, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -211,7 +222,7 @@ int mtp_launches(Model &m, int n, bool head, hipStream_t st) {
     const auto &c = m.c;
     const int H = c.hidden;
     const int64_t abH = act_halves(H);
-    hipLaunchKernelGGL(mtp_in_kernel, dim3(n), dim3(256), 0, st, m.embed, m.sp, m.hbuf, m.mtp_pre_e, m.mtp_pre_h, c.eps,
+    hipLaunchKernelGGL(mtp_in_kernel, dim3(n, 2), dim3(256), 0, st, m.embed, m.sp, m.hbuf, m.mtp_pre_e, m.mtp_pre_h, c.eps,
                        m.mtp_act, act_halves(2 * static_cast<int64_t>(H)));
     GV_CHECK_HIP(hipGetLastError());
     if (gemv_q4(m.mtp_fc, m.mtp_act, act_halves(2 * static_cast<int64_t>(H)), n, gemv_out(m.x, H, m.mtp_fc.global), st) != 0)
@@ -230,7 +241,7 @@ int mtp_launches(Model &m, int n, bool head, hipStream_t st) {
     const int rows = static_cast<int>(hw.rows);
     hipLaunchKernelGGL(pick_max_kernel, dim3(kPickWgs), dim3(kPickThreads), 0, st, m.mtp_logits, rows, pa);
     hipLaunchKernelGGL(pick_sum_kernel, dim3(kPickWgs), dim3(kPickThreads), 0, st, m.mtp_logits, rows,
-                       m.draft_head.rows > 0 ? m.draft_ids : nullptr, pa);
+                       m.draft_head.rows > 0 ? m.draft_ids : nullptr, m.err, pa);
     GV_CHECK_HIP(hipGetLastError());
     return 0;
 }
@@ -272,8 +283,8 @@ int mtp_pass(Model &m, int n, bool head) {
     if (use_act_mode(m.c.exact) != 0) return -1;
     if (mtp_run(m, n, head, st) != 0) return -1;
     const auto *pa = static_cast<const PickArea *>(m.pick);
-    if (head) GV_CHECK_HIP(hipMemcpyAsync(m.pick_host, &pa->draft, 8, hipMemcpyDeviceToHost, st));
-    GV_CHECK_HIP(hipMemcpyAsync(m.pick_host + 2, m.err, 4, hipMemcpyDeviceToHost, st));
+    if (head) GV_CHECK_HIP(hipMemcpyAsync(m.pick_host, &pa->draft, 12, hipMemcpyDeviceToHost, st));   // (with err)
+    else GV_CHECK_HIP(hipMemcpyAsync(m.pick_host + 2, m.err, 4, hipMemcpyDeviceToHost, st));
     GV_CHECK_HIP(hipStreamSynchronize(st));
     GV_REQUIRE(m.pick_host[2] == 0, "MTP pass: a fused launch's wait for its producers ran out (the results are invalid)");
     if (head) m.mtp_last_n = n;
