@@ -352,20 +352,22 @@ __global__ __launch_bounds__(64 * WMAX) void gemv_q4_2pass_kernel(Q4 w, const _F
     }
 }
 
-// The skinny product over many row tiles a workgroup at 17..32 rows (two 16-column tiles: a K range's activations
-// take half the registers, so the kept-parts form above holds only 4 tiles' partial sums and each workgroup reloads
-// the rows' activations every 4 tiles): the waves' sums put every kGemvFlush tiles (mfma_tiles FLUSH), the same
-// sums in the same order as gemv_q4_kernel. A round of the chip's workgroups takes every tile, a stride of the grid
-// apart (all of them read adjacent tiles at a time, at most one tile more than the others), so the activations are
-// loaded once a CU. The waves of the CU's one workgroup (their operands take 8 x 180 registers a lane) wait for one
-// another at a flush only: two halves of the partial sums in turn, one barrier each. PACK 2: at most 24 rows, the
+// The skinny product over many row tiles a workgroup (a vocabulary head): a round of the chip's workgroups takes every
+// tile, a stride of the grid apart (all of them read adjacent tiles at a time, at most one tile more than the others),
+// and the waves' sums are put every few tiles (mfma_tiles FLUSH) with the loads of the next ones in flight: the same
+// sums in the same order as gemv_q4_kernel, the activations loaded once a CU and the partial sums' LDS small. The waves
+// wait for one another at a flush only: two halves of the partial sums in turn, one barrier each; a lane's four rows go
+// out in one store. NTT 2 (17..32 rows): a K range's activations take half the registers; PACK 2: at most 24 rows, the
 // second column tile's hi and lo halves in one MFMA.
-// The 151,936 x 2048 head at 17 rows, with its norm's launch: 62.9 us with four tiles a flush in one buffer over two
+// The 151,936 x 2048 head with its norm's launch, 17 rows: 62.9 us with four tiles a flush in one buffer over two
 // rounds of workgroups; one store a lane 4 rows, packed, two buffers 56.2; one round of workgroups 49.2; two tiles a
 // flush 47.7 (one: 52.5); strided tiles 46.6 (its weights and logits at a copy's rate: 36). Sixteen waves of half the
-// K range each: 58.
-constexpr int kGemvFlush = 2;
-template <int KW, int WMAX, int PACK>
+// K range each: 58. Up to 16 rows against gemv_q4_kernel's contiguous tiles, every tile's sums kept to the end: 1 row
+// 37.9 -> 33.5 us, 5 rows 38.8 -> 35.4, 16 rows 46.7 -> 44.2, 248,320 x 2048 at 5 rows 64.2 -> 54.7, 32,000 x 2048 at 8
+// rows 14.3 -> 13.4; four tiles a flush (eight: the same; two: 2 us more at 16 rows), the ring of three (four: 16 rows
+// spill).
+constexpr int gemv_flush(int ntt) { return ntt == 1 ? 4 : 2; }   // tiles a flush
+template <int KW, int WMAX, int NTT, int PACK>
 __global__ __launch_bounds__(64 * WMAX) void gemv_q4_flush_kernel(Q4 w, const _Float16 *__restrict__ act,
                                                                   int64_t act_stride, int M, int sc0, GemvOut out) {
     extern __shared__ f4 part_lds[];
@@ -377,15 +379,15 @@ __global__ __launch_bounds__(64 * WMAX) void gemv_q4_flush_kernel(Q4 w, const _F
     const bool whole = !out.accumulate && out.nseg == 1 && w.rows % kTileR == 0 &&
                        (reinterpret_cast<uintptr_t>(out.y) | static_cast<uintptr_t>(out.ldy) * 4) % 16 == 0;
     auto tile_of = [&](int i) -> int64_t { return wg + static_cast<int64_t>(i) * nwg; };
-    mfma_tiles<KW, 2, kSplitK, 0, 4, PACK, kGemvFlush, 2>(
+    mfma_tiles<KW, NTT, kSplitK, 0, NTT == 1 ? 3 : 4, PACK, gemv_flush(NTT), 2>(
         w.codes, w.scales, w.rows, static_cast<int>(w.cols / kSuperK), sc0, nt, M,
         [&](int j) { return act + j * act_stride; }, [](int64_t, int, float) {}, part_lds, tab, tile_of, NoHook{},
         NoHook{}, flush_with([&](int i0, int i1, const f4 *part, int W) {   // a tile and column tile a lane: wave order
-            for (int o = threadIdx.x; o < (i1 - i0) * 128; o += blockDim.x) {
-                const int i = o / 128, tt = (o / 64) % 2, ll = o % 64, j = tt * 16 + ll % 16;
+            for (int o = threadIdx.x; o < (i1 - i0) * NTT * 64; o += blockDim.x) {
+                const int i = o / (NTT * 64), tt = (o / 64) % NTT, ll = o % 64, j = tt * 16 + ll % 16;
                 if (j >= M) continue;
-                f4 sum = part[(i * W * 2 + tt) * 64 + ll];
-                for (int w2 = 1; w2 < W; ++w2) sum += part[((i * W + w2) * 2 + tt) * 64 + ll];
+                f4 sum = part[(i * W * NTT + tt) * 64 + ll];
+                for (int w2 = 1; w2 < W; ++w2) sum += part[((i * W + w2) * NTT + tt) * 64 + ll];
                 const int64_t row0 = tile_of(i0 + i) * kTileR + 4 * (ll / 16);
                 if (whole) {
                     *reinterpret_cast<f4 *>(out.y + j * out.ldy + row0) = sum * out.seg_global[0];
@@ -531,21 +533,22 @@ static int launch_gemv(const Q4 &w, const _Float16 *act, int64_t act_stride, int
                        const GemvOut &out, hipStream_t st) {
     const int64_t ntiles = tiles_rows(w.rows);
     const int64_t per = tiles_per_wg(ntiles, waves, NTT);
-    if constexpr (NTT == 2 && !PACK) {
-        // a matrix whose tiles outnumber 4 a workgroup of the chip's resident ones (the head at a tree's 17 rows):
-        // the flushed form, the resident workgroups over all the tiles
-        const int64_t resident = 256 * std::max(1, 8 / waves);
-        if (ntiles > per * resident) {
-            const dim3 grid(static_cast<unsigned>(std::min(ntiles, resident))), block(static_cast<unsigned>(64 * waves));
-            const size_t lds = static_cast<size_t>(2 * kGemvFlush) * waves * NTT * 1024;   // at most 64 KB
-            if (M <= 24)
-                hipLaunchKernelGGL((gemv_q4_flush_kernel<KW, WMAX, 2>), grid, block, lds, st, w, act, act_stride, M, sc0,
-                                   out);
-            else
-                hipLaunchKernelGGL((gemv_q4_flush_kernel<KW, WMAX, 0>), grid, block, lds, st, w, act, act_stride, M, sc0,
-                                   out);
-            return 0;
-        }
+    // a matrix whose tiles outnumber 4 a workgroup of the chip's resident ones (a vocabulary head): the flushed form, the
+    // resident workgroups over all the tiles (up to 16 rows, a range that adds to earlier sums keeps gemv_q4_kernel, which
+    // has those loaded ahead, and so does a traced launch)
+    const int64_t resident = 256 * std::max(1, 8 / waves);
+    const bool flushed = NTT == 1 ? ntiles > 4 * resident && !out.accumulate && out.trace_cls < 0 : ntiles > per * resident;
+    if (flushed) {
+        const dim3 grid(static_cast<unsigned>(std::min(ntiles, resident))), block(static_cast<unsigned>(64 * waves));
+        const size_t lds = static_cast<size_t>(2 * gemv_flush(NTT)) * waves * NTT * 1024;   // at most 64 KB
+        constexpr int P = PACK ? 1 : NTT == 1 ? 0 : 2;
+        if (NTT == 1 || M <= 24)
+            hipLaunchKernelGGL((gemv_q4_flush_kernel<KW, WMAX, NTT, P>), grid, block, lds, st, w, act, act_stride, M, sc0,
+                               out);
+        else
+            hipLaunchKernelGGL((gemv_q4_flush_kernel<KW, WMAX, NTT, NTT == 1 ? P : 0>), grid, block, lds, st, w, act,
+                               act_stride, M, sc0, out);
+        return 0;
     }
     const int64_t wg = (ntiles + per - 1) / per;
     const size_t lds = static_cast<size_t>(per) * waves * NTT * 1024;   // the waves' partial sums

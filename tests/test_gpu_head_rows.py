@@ -1,4 +1,4 @@
-"""The skinny product at 17..32 rows over more row tiles than the chip holds at once (a head's rows): every tile once
+"""The skinny product over more row tiles than the chip holds at once (a head's rows): every tile once
 whatever the tiles leave over a round of workgroups, ragged last tiles, the packed second column tile's edge (24 rows),
 narrow K (several workgroups a CU) and K in two ranges (the second adds to the first's sums)."""
 import numpy as np
@@ -11,6 +11,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("rows,cols,M,add", [
     (16400, 2048, 17, False), (16401, 2048, 24, False), (16640, 2048, 25, False), (32771, 2048, 32, False),
+    (16400, 2048, 1, False), (16401, 2048, 8, False), (32784, 2048, 9, False), (32771, 2048, 16, False),
+    (16400, 6144, 5, False), (65552, 512, 4, False), (131104, 128, 3, False), (17000, 2048, 5, True),
     (70000, 512, 17, False), (131104, 128, 18, True), (20496, 4096, 24, False), (17000, 2048, 17, True)])
 def test_gemv_many_tiles(rows, cols, M, add):
     import geode_amd as gv
