@@ -77,7 +77,7 @@ __device__ inline int pick_chunk(int rows) { return (rows + kPickWgs - 1) / kPic
 
 // The maximum: per chunk its largest logit and first index (sc1 stores), then the last workgroup to finish takes the
 // chunks, a lane each (the largest value, of equal ones the lowest index: the first maximum), into maxv / best. Bound by
-// the chain launch, chunk, hand-off, chunks: 32,000 rows 10.9 us with one thread over the chunks, 4.8 so.
+// the chain launch, chunk, hand-off, chunks: 32,768 rows 10.9 us with one thread over the chunks, 4.8 so.
 __global__ __launch_bounds__(kPickThreads) void pick_max_kernel(const float *__restrict__ lg, int rows, PickArea *pa) {
     __shared__ float sv[kPickThreads / 64];
     __shared__ int si[kPickThreads / 64];
@@ -112,7 +112,7 @@ __global__ __launch_bounds__(kPickThreads) void pick_max_kernel(const float *__r
 
 // The probability: per chunk sum exp(double(l - max)) (the difference in fp32 as the reference's, softmax_at), then the
 // last workgroup adds the chunks' sums in order (read a lane each): prob = 1 / sum, draft = the best index (through ids
-// when a draft vocabulary is set). 32,000 rows: 6.2 us with one thread reading the sums, 4.9 so.
+// when a draft vocabulary is set). 32,768 rows: 6.2 us with one thread reading the sums, 4.9 so.
 __global__ __launch_bounds__(kPickThreads) void pick_sum_kernel(const float *__restrict__ lg, int rows,
                                                                 const int32_t *__restrict__ ids,
                                                                 const int *__restrict__ err, PickArea *pa) {
