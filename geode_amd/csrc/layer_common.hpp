@@ -53,18 +53,10 @@ __host__ __device__ inline int attn_k_ld(int hd) { return hd + 8; }   // halves 
 constexpr int kAttnVld = kAttnBlock + 8;                              // halves a staged value row
 inline size_t attn_lds(int hd) { return (static_cast<size_t>(kAttnBlock) * attn_k_ld(hd) + hd * kAttnVld) * 2; }
 
-// The attention's split (attn_block_kernel): the groups of up to four 16-query tiles a KV head's queries make, the
-// blocks a workgroup takes one after the other (its run) - one until all the blocks' workgroups pass kAttnUnits, two a
-// CU, then as many as keep them below it - and the runs, the partials of a (row, head). nkv_groups: n_kv_heads x groups.
-constexpr int kAttnUnits = 512;
+// The groups of up to four 16-query tiles that a KV head's queries make, a workgroup of attn_block_kernel each while the
+// (block, KV head) units are at most kAttnGroupUnits a group; past that a unit's one workgroup takes them all.
+constexpr int kAttnGroupUnits = 100;
 __host__ __device__ inline int attn_groups(int nh, int nkv, int M) { return (nh / nkv * M + 63) / 64; }
-__host__ __device__ inline int attn_run_blocks(int nb, int nkv_groups) {
-    return (nb * nkv_groups + kAttnUnits - 1) / kAttnUnits;
-}
-__host__ __device__ inline int attn_runs(int total, int nkv_groups) {
-    const int nb = (total + kAttnBlock - 1) / kAttnBlock, R = attn_run_blocks(nb, nkv_groups);
-    return (nb + R - 1) / R;
-}
 
 // route_topk (model.cpp:4021-4065) of NR rows by one wave, the rows' dependency chains interleaved: softmax over the
 // E <= 256 experts (max, expf, the sum, divide), the top K by probability with ties to the lower index, the weights

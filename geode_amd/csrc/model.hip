@@ -130,29 +130,28 @@ __global__ __launch_bounds__(256) void qk_rope_kernel(const float *__restrict__ 
 }
 
 
-// Split-KV attention on the matrix cores: a workgroup (4 waves) per (run of blocks of 64 positions, KV head, group of
-// up to four tiles of 16 queries), a wave a query tile (the KV head's query heads x the rows). Block by block the keys
-// [64][hd] and values [hd][64] are staged in LDS by all the threads (positions past the context as zeros), then
-// S^T = K Q^T (v_mfma_f32_16x16x32_f16: fp16 keys, the queries as hi + lo fp16 halves, fp32 sums), masked to the
-// context plus each row's visible rows, the weights exp(s - the run's maximum so far) and their sum;
-// O^T = V^T P^T with the weights as hi + lo halves, the earlier blocks' values scaled to the new maximum. Writes the
-// run's partial (weighted values, max, sum) as attend_heads does per block (model.cpp:3894-4018); attn_merge joins
-// them. A run of one block is that block's own partial, bit for bit.
+// Split-KV attention on the matrix cores: a workgroup (4 waves) per (block of 64 positions, KV head, group of tiles of 16
+// queries), a wave a query tile after the other (the KV head's query heads x the rows). The block's keys [64][hd] and
+// values [hd][64] are staged in LDS by all the threads (positions past the context as zeros), then S^T = K Q^T
+// (v_mfma_f32_16x16x32_f16: fp16 keys, the queries as hi + lo fp16 halves, fp32 sums), masked to the context plus each
+// row's visible rows, then per query the block's maximum, the weights exp(s - max) and their sum; O^T = V^T P^T with
+// the weights as hi + lo halves. Writes the block's partial (weighted values, max, sum) as attend_heads does per block
+// (model.cpp:3894-4018); attn_merge joins them. What a row gives depends on its context alone, not on how many rows or
+// positions the step has.
 //
-// A block a workgroup until the workgroups fill the chip twice (attn_run_blocks: two a CU, 70 KB of LDS each, one
-// staging while the other computes), then runs: what a long context or a tree costs is mostly the partials, a float a
-// (query, dim) and run written here and read by the merge (17 rows over 32,000 positions: 140 MB in blocks, 23 MB in
-// runs of six, against 33 MB of int8 keys and values). This and the merge: 17 rows over 32,001 int8 positions 93 us in
-// blocks, 48 in runs; 17 rows over 8,192 fp16 positions 34 and 27; 5 rows over 8,192 (blocks) 18.4. A run is bound by
-// the waves' vector instructions (the weights' exponentials and their hi + lo split, the int8 keys and values made
-// fp16), two waves a SIMD at 250 registers: hence 2^x of scores in units of log 2, one mask test a block, the values
-// summed in place.
+// Bound by its vector work (the weights' exponentials and hi + lo split, the int8 operands made fp16) and, over long
+// contexts and many rows, by the partials: a float a (query, dim) and block written here and read by the merge (17 rows
+// over 32,000 positions: 140 MB against 33 MB of int8 keys and values). Several blocks a workgroup with one partial
+// (42 us with the merge there, 92 so) were taken back: their sums over the blocks depend on how the step is split and
+// are rounded again where a maximum moves, and so were weights as 2^x of scores in units of log 2 (one instruction a
+// score less), which round every score once more: at scores of 2,000 a weight is off by 1e-4 instead of 1e-7.
+// Groups: a unit of many tiles takes as many turns as its waves need; in groups the turns are one, but every group
+// stages the block again, so they pay only while the chip has room (kAttnGroupUnits: head_dim 256, 2 KV heads, fp16, 17
+// rows in three groups or one: 2,048 positions 9.1 or 16.3 us, 8,192 20.4 or 24.2, 12,000 29.7 or 25.9; 9 rows in two
+// groups or one: 4,096 positions 11.6 or 12.2, 8,192 17.4 or 16.2).
+// int8: two workgroups a CU asked for (160 registers; 17 rows over 32,000 positions 54 us, 55.6 without); fp16 without
+// (9 rows over 16,000: 20.5 us, 23.7 with).
 
-// NCH = head_dim / 32: every loop over the head's dims, and every load, fixed at compile time (no branch around a
-// load, so the compiler waits for exactly the loads each step needs)
-// I8: the int8 cache (attend<int8_t>): keys and values staged as fp16 (the int8 values, exact), the block's K and V
-// scales in LDS; a score is the dot times (1 / sqrt(hd)) x the position's K scale (model.cpp:3948), the weights'
-// sum is the softmax's own and each weight then takes the position's V scale before the values (:3965-3972).
 // 8 int8 values (little-endian) as fp16: a byte + 128 as the low bits of the fp16 1024, then - 1152 (exact)
 __device__ inline half8 i8_to_h8(uint32_t lo, uint32_t hi) {
     typedef _Float16 half2v __attribute__((ext_vector_type(2)));
@@ -170,27 +169,49 @@ __device__ inline half8 i8_to_h8(uint32_t lo, uint32_t hi) {
     return __builtin_bit_cast(half8, u4v{o[0], o[1], o[2], o[3]});
 }
 
-// The unit's work: blocks [b0, b1) of the KV head kh for the query group qg, the partial to place `run`. RUNS false: one
-// block (b1 = b0 + 1), whose values go out as they are made, nothing kept.
-struct AttnUnit {
-    int kh, qg, run, b0, b1;
-};
-template <int NCH, bool I8, bool RUNS>
-__device__ inline void attn_unit(const _Float16 *__restrict__ q16, const void *__restrict__ kvp,
-                                 const float *__restrict__ kvs, int64_t slots, int nh, int nkv,
-                                 const StepParams *__restrict__ sp, float *__restrict__ parts, int nb_max, int G,
-                                 const AttnUnit un, _Float16 *lds_h, float *sc_l) {
+// NCH = head_dim / 32: every loop over the head's dims, and every load, fixed at compile time (no branch around a
+// load, so the compiler waits for exactly the loads each step needs)
+// I8: the int8 cache (attend<int8_t>): keys and values staged as fp16 (the int8 values, exact), the block's K and V
+// scales in LDS; a score is the dot times (1 / sqrt(hd)) x the position's K scale (model.cpp:3948), the weights'
+// sum is the softmax's own and each weight then takes the position's V scale before the values (:3965-3972).
+// G: the groups (attn_groups)
+template <int NCH, bool I8>
+__global__ __launch_bounds__(256, I8 ? 2 : 1) void attn_block_kernel(const _Float16 *__restrict__ q16,
+                                                            const void *__restrict__ kvp,
+                                                            const float *__restrict__ kvs, int64_t slots, int nh,
+                                                            int nkv, const StepParams *__restrict__ sp,
+                                                            float *__restrict__ parts, int nb_max, int G) {
     constexpr int hd = NCH * 32;
-    const int pos = sp->pos, M = sp->M, total = pos + M, kh = un.kh;
+    extern __shared__ _Float16 lds_h[];
+    __shared__ __align__(16) float sc_l[I8 ? 256 : 4];   // int8: the block's K scales [0, 64), V scales [64, 128)
+    trace(GV_K_ATTN, 0);
+    const int pos = sp->pos, M = sp->M, total = pos + M;
+    // workgroup i -> (unit, query group): a unit's groups are 8 apart, so on one XCD (its L2 then serves the second
+    // group's keys and values); unit -> (block, KV head): the context's last block (usually a few new rows) of every KV
+    // head takes the highest units, so that the workgroups past one a CU, dispatched last, are those short ones
+    const int nb_live = (total + kAttnBlock - 1) / kAttnBlock;
+    const bool split = G > 1 && nb_live * nkv <= kAttnGroupUnits * G;
+    const int wi = split ? static_cast<int>(blockIdx.x / (8 * G)) * 8 + static_cast<int>(blockIdx.x % 8)
+                         : static_cast<int>(blockIdx.x);
+    const int groups = split ? G : 1, gi = split ? static_cast<int>(blockIdx.x / 8) % G : 0;
+    if (wi >= nb_live * nkv) return;
+    // (divisions leave uniform values in vector registers: into scalar ones, so that the block's addresses are)
+    auto uni = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
+    const int b = uni(wi < (nb_live - 1) * nkv ? wi / nkv : nb_live - 1);
+    const int kh = uni(wi < (nb_live - 1) * nkv ? wi % nkv : wi - (nb_live - 1) * nkv);
+    const int s0 = b * kAttnBlock;
+    const int live = total - s0;   // positions of the block inside the context (1 .. 64, or more)
     const int kld = attn_k_ld(hd);
     _Float16 *ks = lds_h, *vs = lds_h + kAttnBlock * kld;
-    const int group = __builtin_amdgcn_readfirstlane(nh / nkv), NQ = group * M, nqt = (NQ + 15) / 16;
+    const int group = uni(nh / nkv), NQ = group * M, nqt = (NQ + 15) / 16;
     const int wave = threadIdx.x / 64, l = threadIdx.x % 64, lq = l % 16, lg = l / 16;
     const int64_t qlo = static_cast<int64_t>(M) * nh * hd;
+    // the group's tiles [gi tg, qt1), wave w's the w-th of every four
+    const int tg = (nqt + groups - 1) / groups, qt0 = uni(gi * tg + wave), qt1 = uni(min(gi * tg + tg, nqt));
     // the queries of tile qt as B operands (hi and lo halves): dims ch * 32 + 8 lg .. + 8 of query qt * 16 + lq
-    auto load_q = [&](int qt, half8 (&qb)[NCH], half8 (&ql)[NCH]) {
-        // (a query past the tile's end reads query 0: its scores are masked and its output is not written, so
-        // nothing waits on a select of the loaded values)
+    half8 qb[NCH], ql[NCH];
+    auto load_q = [&](int qt) {
+        // (a query past the last reads query 0 and is not written: nothing waits on a select of the loaded values)
         const int qi = qt * 16 + lq;
         const bool ok = qi < NQ;
         const int tq = ok ? qi / group : 0, hq = kh * group + (ok ? qi % group : 0);
@@ -201,45 +222,18 @@ __device__ inline void attn_unit(const _Float16 *__restrict__ q16, const void *_
             ql[ch] = *reinterpret_cast<const half8 *>(qp + qlo + ch * 32);
         }
     };
-    // the wave's tile of queries
-    const int tg = __builtin_amdgcn_readfirstlane((nqt + G - 1) / G);
-    const int qt = __builtin_amdgcn_readfirstlane(un.qg * tg + wave);
-    const bool active = wave < tg && qt < nqt;
-    half8 qb[NCH], ql[NCH];
-    load_q(qt, qb, ql);   // in flight with the staging loads
-    // the visibility mask of the lane's query row (sp->vis: bit j = the row sees new row j), loaded with them
-    const bool qvalid = active && qt * 16 + lq < NQ;
-    const uint32_t vis = sp->vis[min((qt * 16 + lq) / group, M - 1)];
-    // 1 / sqrt(hd) x log2(e): the scores in units of log 2, so that the weights are the hardware's 2^x (1 ulp) with no
-    // product of their own; a score's rounding is the same share of it either way
-    const float scale = __uint_as_float(__builtin_amdgcn_readfirstlane(   // (uniform: a scalar register)
-        __float_as_uint(__fmul_rn(__fdiv_rn(1.0f, __fsqrt_rn(static_cast<float>(hd))), 1.44269504088896341f))));
-    constexpr int NDT = hd / 16;   // 16-dim tiles of the head (2 NCH: not always a multiple of four)
-    float4v O[RUNS ? NDT : 1];   // the run's weighted values, O^T[dim dt*16 + 4 lg + r][query lq], relative to its maximum mrun
-    float mrun = -__builtin_inff(), lrun = 0.0f;
-#pragma unroll
-    for (int dt = 0; dt < (RUNS ? NDT : 1); ++dt) O[dt] = float4v{0, 0, 0, 0};
-    // the partial of query lane % 16 of the wave's tile (the lane made anew, as in the loop)
-    auto part_of = [&](int tid) {
-        int grp = nh / nkv;   // (made anew: what dividing by it takes is not kept over the run either)
-        if constexpr (RUNS) asm volatile("" : "+v"(grp));
-        const int qi = min(qt * 16 + tid % 16, NQ - 1);
-        return parts + ((static_cast<int64_t>(qi / grp) * nh + kh * grp + qi % grp) * nb_max + un.run) * (hd + 2);
-    };
-    float *dst = nullptr;
-    if constexpr (!RUNS) dst = part_of(threadIdx.x);
-    // the int8 cache's loads of a block (every one issued before the first use): a run's next block's are in flight while
-    // the current one is computed
-    constexpr int nld8 = kAttnBlock * hd / 16, nl8 = (nld8 + 255) / 256;   // 16-byte loads of K (and of V), a thread's
-    u4v kr8[I8 ? nl8 : 1], vr8[I8 ? nl8 : 1];
-    float scv8 = 0.0f;   // thread j < 64: the K scale of position j, 64 <= j < 128: the V scale
-    auto load8 = [&](int b, int tid, u4v (&kr)[I8 ? nl8 : 1], u4v (&vr)[I8 ? nl8 : 1], float &scv) {
-        const int s0 = b * kAttnBlock, live = total - s0;
+    load_q(qt0);   // the wave's first tile of queries, in flight with the staging loads
+    // the visibility masks of the lane's query rows (sp->vis: bit j = the row sees new row j), loaded with them
+    auto vis_of = [&](int qt) { return sp->vis[min((qt * 16 + lq) / group, M - 1)]; };
+    uint32_t vis = vis_of(qt0);
+    if constexpr (I8) {   // int8: a block's K (or V) is 64 x hd bytes, 16 a load; fp16 in the LDS
         const char *kg = static_cast<const char *>(kvp) + k_index(slots, hd, kh, s0, 0);
         const char *vg = static_cast<const char *>(kvp) + v_index(slots, hd, nkv, kh, s0, 0);
+        constexpr int nld = kAttnBlock * hd / 16, nl = (nld + 255) / 256;   // 16-byte loads of each, a thread's
+        u4v kr[nl], vr[nl];
 #pragma unroll
-        for (int u = 0; u < (I8 ? nl8 : 1); ++u) {
-            const int i = min(tid + u * 256, nld8 - 1);
+        for (int u = 0; u < nl; ++u) {
+            const int i = min(static_cast<int>(threadIdx.x) + u * 256, nld - 1);
             // (rows past the context read the last live row again, from the cache: their scores are masked and their
             // weights zero; 32-bit offsets from the block's base: one register a load)
             const int kr_row = min(i / (hd / 16), live - 1);
@@ -247,69 +241,49 @@ __device__ inline void attn_unit(const _Float16 *__restrict__ q16, const void *_
             const int vd = i / (kAttnBlock / 16), vc = min(i % (kAttnBlock / 16), (live - 1) / 16);
             vr[u] = *reinterpret_cast<const u4v *>(vg + static_cast<uint32_t>((vd * (kAttnBlock / 16) + vc) * 16));
         }
-        scv = kvs[kv_scale_index(slots, nkv, (tid / kAttnBlock) & 1, kh, s0 + tid % kAttnBlock)];
+        // the block's scales: thread j < 64 the K scale of position j, 64 <= j < 128 the V scale (0 past the
+        // context, so that a weight 0 stays 0)
+        const int j = threadIdx.x % kAttnBlock, which = (threadIdx.x / kAttnBlock) & 1;
+        const float scv = kvs[kv_scale_index(slots, nkv, which, kh, s0 + j)];
         __builtin_amdgcn_sched_barrier(0);
-    };
-    if constexpr (I8) load8(un.b0, threadIdx.x, kr8, vr8, scv8);
-    for (int b = un.b0; b < (RUNS ? un.b1 : un.b0 + 1); ++b) {
-    const int s0 = b * kAttnBlock;
-    const int live = total - s0;   // positions of the block inside the context (1 .. 64, or more)
-    // (the thread's index made anew each block, so that the addresses made from it are not kept in registers over the
-    // whole run: with them the wave's queries and values would not fit 256)
-    int tid = threadIdx.x;
-    if constexpr (RUNS) asm volatile("" : "+v"(tid));
-    if (RUNS && b > un.b0) __syncthreads();   // (the previous block's operands have been read)
-    if constexpr (I8) {   // a block's K (or V) is 64 x hd bytes, 16 a load; fp16 in the LDS
 #pragma unroll
-        for (int u = 0; u < nl8; ++u) {   // (a thread past nld8 stores item nld8 - 1 again: no branch to sink loads into)
-            const int i = min(tid + u * 256, nld8 - 1);
+        for (int u = 0; u < nl; ++u) {   // (a thread past nld stores item nld - 1 again: no branch to sink loads into)
+            const int i = min(static_cast<int>(threadIdx.x) + u * 256, nld - 1);
             const int r = i / (hd / 16), c = i % (hd / 16);
-            *reinterpret_cast<half8 *>(ks + r * kld + c * 16) = i8_to_h8(kr8[u].x, kr8[u].y);
-            *reinterpret_cast<half8 *>(ks + r * kld + c * 16 + 8) = i8_to_h8(kr8[u].z, kr8[u].w);
+            *reinterpret_cast<half8 *>(ks + r * kld + c * 16) = i8_to_h8(kr[u].x, kr[u].y);
+            *reinterpret_cast<half8 *>(ks + r * kld + c * 16 + 8) = i8_to_h8(kr[u].z, kr[u].w);
             const int d = i / (kAttnBlock / 16), cv = i % (kAttnBlock / 16);
-            *reinterpret_cast<half8 *>(vs + d * kAttnVld + cv * 16) = i8_to_h8(vr8[u].x, vr8[u].y);
-            *reinterpret_cast<half8 *>(vs + d * kAttnVld + cv * 16 + 8) = i8_to_h8(vr8[u].z, vr8[u].w);
+            *reinterpret_cast<half8 *>(vs + d * kAttnVld + cv * 16) = i8_to_h8(vr[u].x, vr[u].y);
+            *reinterpret_cast<half8 *>(vs + d * kAttnVld + cv * 16 + 8) = i8_to_h8(vr[u].z, vr[u].w);
         }
-        // (the V scale 0 past the context, so that a weight 0 stays 0; threads >= 128: copies, unused)
-        sc_l[tid] = ((tid / kAttnBlock) & 1) == 1 && s0 + tid % kAttnBlock >= total ? 0.0f : scv8;
+        sc_l[threadIdx.x] = which == 1 && s0 + j >= total ? 0.0f : scv;   // (threads >= 128: copies, unused)
     } else {   // stage: keys row by row, values (already [hd][64] in the cache) row by row; 8 halves a load, every
                // load of the thread issued before the first store (NCH of each)
-        const _Float16 *kv = static_cast<const _Float16 *>(kvp);
-        const _Float16 *kg = kv + k_index(slots, hd, kh, s0, 0);
-        const _Float16 *vg = kv + v_index(slots, hd, nkv, kh, s0, 0);
         // (byte offsets in 32 bits from the block's uniform bases: one register a load)
-        const char *kb8 = reinterpret_cast<const char *>(kg), *vb8 = reinterpret_cast<const char *>(vg);
+        const _Float16 *kv = static_cast<const _Float16 *>(kvp);
+        const char *kg = reinterpret_cast<const char *>(kv + k_index(slots, hd, kh, s0, 0));
+        const char *vg = reinterpret_cast<const char *>(kv + v_index(slots, hd, nkv, kh, s0, 0));
         const int kpr = hd / 8;   // loads a key row
         const int nl = hd / 32;   // loads a thread of each
         u4v kr[8], vr[8];   // (native vectors: an array of HIP's struct type may be kept in scratch)
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
             if (u >= nl) break;
-            const int i = tid + u * 256;
+            const int i = threadIdx.x + u * 256;
             const int r = i / kpr, c = i % kpr;
             // (rows past the context read the last live row again, from the cache: their scores are masked; values
             // past it are zeroed below, as a weight 0 times a stale non-finite value would not be 0, and their
             // 8-position pieces past the last live one read that one again)
-            kr[u] = *reinterpret_cast<const u4v *>(kb8 + static_cast<uint32_t>((min(r, live - 1) * hd + c * 8) * 2));
+            kr[u] = *reinterpret_cast<const u4v *>(kg + static_cast<uint32_t>((min(r, live - 1) * hd + c * 8) * 2));
             const int vd = i / (kAttnBlock / 8), vc = min(i % (kAttnBlock / 8), (live - 1) / 8);
-            vr[u] = *reinterpret_cast<const u4v *>(vb8 + static_cast<uint32_t>((vd * (kAttnBlock / 8) + vc) * 16));
-            if constexpr (RUNS) __builtin_amdgcn_sched_barrier(0);   // (one load's address at a time)
+            vr[u] = *reinterpret_cast<const u4v *>(vg + static_cast<uint32_t>((vd * (kAttnBlock / 8) + vc) * 16));
         }
         __builtin_amdgcn_sched_barrier(0);   // every load issued before the first store waits for one
-        if constexpr (RUNS) {   // (the keys' registers free before the values' masks are made)
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                if (u >= nl) break;
-                const int i = tid + u * 256;
-                *reinterpret_cast<u4v *>(ks + (i / kpr) * kld + (i % kpr) * 8) = kr[u];
-            }
-            __builtin_amdgcn_sched_barrier(0);
-        }
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
             if (u >= nl) break;
-            const int i = tid + u * 256;
-            if constexpr (!RUNS) *reinterpret_cast<u4v *>(ks + (i / kpr) * kld + (i % kpr) * 8) = kr[u];
+            const int i = threadIdx.x + u * 256;
+            *reinterpret_cast<u4v *>(ks + (i / kpr) * kld + (i % kpr) * 8) = kr[u];
             const int d = i / (kAttnBlock / 8), cv = i % (kAttnBlock / 8);
             const int lim = live - cv * 8;   // positions of this load inside the context
             auto keep = [&](int k) {   // the word's halves (positions 2k, 2k + 1) inside the context: kept (no branch:
@@ -318,18 +292,20 @@ __device__ inline void attn_unit(const _Float16 *__restrict__ q16, const void *_
             };
             const u4v v = {vr[u].x & keep(0), vr[u].y & keep(1), vr[u].z & keep(2), vr[u].w & keep(3)};
             *reinterpret_cast<u4v *>(vs + d * kAttnVld + cv * 8) = v;
-            if constexpr (RUNS) __builtin_amdgcn_sched_barrier(0);
         }
     }
     __syncthreads();
-    if constexpr (I8 && RUNS) load8(min(b + 1, un.b1 - 1), tid, kr8, vr8, scv8);   // (the last: itself again, unused)
-    if constexpr (!RUNS) trace(GV_K_ATTN, 1);
-    if (active) {
-        const int lq = tid % 16, lg = (tid % 64) / 16;
+    trace(GV_K_ATTN, 1);
+    const float scale = __fdiv_rn(1.0f, __fsqrt_rn(static_cast<float>(hd)));
+    for (int qt = qt0; qt < qt1; qt += 4) {
+        if (qt != qt0) load_q(qt), vis = vis_of(qt);
+        const int qi = qt * 16 + lq;
+        const bool qvalid = qi < NQ;
+        const int tq = qvalid ? qi / group : 0, hq = kh * group + (qvalid ? qi % group : 0);
         // the four 16-position tiles' scores, hi and lo products apart: eight independent MFMA chains. The keys'
         // operands come from LDS a group of KG chunks at a time, the next group's reads issued before the current
         // group's products (double-buffered), so that no product waits for a read issued just before it
-        constexpr int KG = RUNS ? 1 : 2, NKG = (NCH + KG - 1) / KG;
+        constexpr int KG = 2, NKG = (NCH + KG - 1) / KG;
         float4v ch_[4], cl_[4];
 #pragma unroll
         for (int pt = 0; pt < 4; ++pt) ch_[pt] = cl_[pt] = float4v{0, 0, 0, 0};
@@ -358,7 +334,7 @@ __device__ inline void attn_unit(const _Float16 *__restrict__ q16, const void *_
                 }
             __builtin_amdgcn_sched_barrier(0);
         }
-        float sc[4][4];   // S^T[position pt*16 + 4 lg + r][query lq], in units of log 2
+        float sc[4][4];   // S^T[position pt*16 + 4 lg + r][query lq]
 #pragma unroll
         for (int pt = 0; pt < 4; ++pt) {
             float4v kf = {scale, scale, scale, scale};
@@ -380,14 +356,9 @@ __device__ inline void attn_unit(const _Float16 *__restrict__ q16, const void *_
         float mx = sc[0][0];
 #pragma unroll
         for (int i = 1; i < 16; ++i) mx = fmaxf(mx, sc[i / 4][i % 4]);
-        if constexpr (!RUNS) trace(GV_K_ATTN, 2);
+        if (qt == qt0) trace(GV_K_ATTN, 2);
         mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
         mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-        mx = fmaxf(mx, mrun);
-        // (the run's first block with a visible position: the sums so far are zeros)
-        const float alpha = mrun == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f(mrun - mx);
-        mrun = mx;
-        const float mref = mx == -__builtin_inff() ? 0.0f : mx;   // (nothing visible yet: the weights are exp(-inf))
         float lsum = 0.0f;
         half4 pe[4], pl[4];   // the weights as hi + lo halves
 #pragma unroll
@@ -396,7 +367,7 @@ __device__ inline void attn_unit(const _Float16 *__restrict__ q16, const void *_
             if constexpr (I8) vf = *reinterpret_cast<const float4v *>(sc_l + kAttnBlock + pt * 16 + 4 * lg);
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const float e = __builtin_amdgcn_exp2f(sc[pt][r] - mref);   // (masked: 0)
+                const float e = sc[pt][r] == -__builtin_inff() ? 0.0f : expf(sc[pt][r] - mx);
                 _Float16 eh, el;
                 split_f16(I8 ? e * vf[r] : e, eh, el);
                 pe[pt][r] = eh;
@@ -406,7 +377,6 @@ __device__ inline void attn_unit(const _Float16 *__restrict__ q16, const void *_
         }
         lsum += __shfl_xor(lsum, 16, 64);
         lsum += __shfl_xor(lsum, 32, 64);
-        lrun = __builtin_fmaf(lrun, alpha, lsum);
         // P^T operands of the two 32-position chunks: k-slot j < 4 is position 32 kc + 4 lg + j, j >= 4 is
         // 32 kc + 16 + 4 lg + j - 4; the V^T operands take the same positions
         half8 pb[2], pbl[2];
@@ -419,22 +389,18 @@ __device__ inline void attn_unit(const _Float16 *__restrict__ q16, const void *_
                 pbl[kc][j] = pl[2 * kc][j];
                 pbl[kc][4 + j] = pl[2 * kc + 1][j];
             }
-        if constexpr (RUNS) {
-            if (!__all(alpha == 1.0f)) {   // (uniform: a maximum moved)
-#pragma unroll
-                for (int dt = 0; dt < NDT; ++dt) O[dt] *= alpha;
-            }
-        }
-        constexpr int VT = RUNS ? 2 : 4, NVG = (NDT + VT - 1) / VT;   // dim tiles at a time (fewer where O is kept)
-        // the values' operands of VT 16-dim tiles (both 32-position chunks), read a group ahead like the keys'
-        half8 vb[2][2][VT];
-        auto load_v = [&](int vg, half8 (&dstv)[2][VT]) {
+        float *dst = parts + ((static_cast<int64_t>(tq) * nh + hq) * nb_max + b) * (hd + 2);
+        constexpr int NDT = hd / 16;   // 16-dim tiles of the head (2 NCH: not always a multiple of four)
+        constexpr int NVG = (NDT + 3) / 4;
+        // the values' operands of four 16-dim tiles (both 32-position chunks), read a group ahead like the keys'
+        half8 vb[2][2][4];
+        auto load_v = [&](int vg, half8 (&dstv)[2][4]) {
 #pragma unroll
             for (int kc = 0; kc < 2; ++kc)
 #pragma unroll
-                for (int k = 0; k < VT; ++k) {
-                    if (VT * vg + k >= NDT) continue;   // (compile time)
-                    const _Float16 *vrow = vs + ((VT * vg + k) * 16 + lq) * kAttnVld;
+                for (int k = 0; k < 4; ++k) {
+                    if (4 * vg + k >= NDT) continue;   // (compile time)
+                    const _Float16 *vrow = vs + ((4 * vg + k) * 16 + lq) * kAttnVld;
                     const half4 lo = *reinterpret_cast<const half4 *>(vrow + kc * 32 + 4 * lg);
                     const half4 hi = *reinterpret_cast<const half4 *>(vrow + kc * 32 + 16 + 4 * lg);
                     dstv[kc][k] = half8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
@@ -442,86 +408,35 @@ __device__ inline void attn_unit(const _Float16 *__restrict__ q16, const void *_
         };
         load_v(0, vb[0]);
 #pragma unroll
-        for (int vg = 0; vg < NVG; ++vg) {   // hi and lo apart: 2 VT independent MFMA chains
-            const int dt0 = VT * vg;
+        for (int vg = 0; vg < NVG; ++vg) {   // four 16-dim tiles at a time, hi and lo apart
+            const int dt0 = 4 * vg;
             if (vg + 1 < NVG) load_v(vg + 1, vb[(vg + 1) & 1]);
             __builtin_amdgcn_sched_barrier(0);
-            if constexpr (RUNS) {   // onto the run's values
+            float4v oh[4], ol[4];
 #pragma unroll
-                for (int kc = 0; kc < 2; ++kc)
-#pragma unroll
-                    for (int h = 0; h < 2; ++h)
-#pragma unroll
-                        for (int k = 0; k < VT; ++k)
-                            O[dt0 + k] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vb[vg & 1][kc][k], h ? pbl[kc] : pb[kc],
-                                                                                O[dt0 + k], 0, 0, 0);
-                continue;
-            }
-            float4v oh[VT], ol[VT];
-#pragma unroll
-            for (int k = 0; k < VT; ++k) oh[k] = ol[k] = float4v{0, 0, 0, 0};
+            for (int k = 0; k < 4; ++k) oh[k] = ol[k] = float4v{0, 0, 0, 0};
 #pragma unroll
             for (int kc = 0; kc < 2; ++kc)
 #pragma unroll
-                for (int k = 0; k < VT; ++k) {
+                for (int k = 0; k < 4; ++k) {
                     if (dt0 + k >= NDT) break;   // (compile time: the loops are unrolled)
                     oh[k] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vb[vg & 1][kc][k], pb[kc], oh[k], 0, 0, 0);
                     ol[k] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vb[vg & 1][kc][k], pbl[kc], ol[k], 0, 0, 0);
                 }
 #pragma unroll
-            for (int k = 0; k < VT; ++k) {   // O^T[dim dt*16 + 4 lg + r][query lq]
+            for (int k = 0; k < 4; ++k) {   // O^T[dim dt*16 + 4 lg + r][query lq]
                 if (dt0 + k >= NDT) break;
                 const float4v c = oh[k] + ol[k];
                 if (qvalid)
                     *reinterpret_cast<float4 *>(dst + (dt0 + k) * 16 + 4 * lg) = make_float4(c[0], c[1], c[2], c[3]);
             }
         }
-    }
-    }
-    if (qvalid) {
-        int tid = threadIdx.x;
-        if constexpr (RUNS) {
-            asm volatile("" : "+v"(tid));
-            dst = part_of(tid);
-#pragma unroll
-            for (int dt = 0; dt < NDT; ++dt)
-                *reinterpret_cast<float4 *>(dst + dt * 16 + 4 * ((tid % 64) / 16)) =
-                    make_float4(O[dt][0], O[dt][1], O[dt][2], O[dt][3]);
+        if (qvalid && lg == 0) {
+            dst[hd] = mx;
+            dst[hd + 1] = lsum;
         }
-        if (tid % 64 < 16) {
-            dst[hd] = mrun;
-            dst[hd + 1] = lrun;
-        }
+        if (qt == qt0) trace(GV_K_ATTN, 3);
     }
-    trace(GV_K_ATTN, 3);
-}
-
-template <int NCH, bool I8>
-__global__ __launch_bounds__(256, 2) void attn_block_kernel(const _Float16 *__restrict__ q16,
-                                                            const void *__restrict__ kvp,
-                                                            const float *__restrict__ kvs, int64_t slots, int nh,
-                                                            int nkv, const StepParams *__restrict__ sp,
-                                                            float *__restrict__ parts, int nb_max, int G) {
-    extern __shared__ _Float16 lds_h[];
-    __shared__ __align__(16) float sc_l[I8 ? 256 : 4];   // int8: the block's K scales [0, 64), V scales [64, 128)
-    trace(GV_K_ATTN, 0);
-    const int total = sp->pos + sp->M;
-    // workgroup i -> (unit, query group): a unit's groups are 8 apart, so on one XCD (its L2 then serves the second
-    // group's keys and values); unit -> (run, KV head): the context's last run (usually a few new rows) of every KV
-    // head takes the highest units, so that the workgroups past one a CU, dispatched last, are those short ones
-    const int nb = (total + kAttnBlock - 1) / kAttnBlock, R = attn_run_blocks(nb, nkv * G), nr = (nb + R - 1) / R;
-    const int wi = G == 1 ? static_cast<int>(blockIdx.x)
-                          : static_cast<int>(blockIdx.x / (8 * G)) * 8 + static_cast<int>(blockIdx.x % 8);
-    const int qg = G == 1 ? 0 : static_cast<int>(blockIdx.x / 8) % G;
-    if (wi >= nr * nkv) return;
-    const int run = wi < (nr - 1) * nkv ? wi / nkv : nr - 1;
-    const int kh = wi < (nr - 1) * nkv ? wi % nkv : wi - (nr - 1) * nkv;
-    // (divisions leave uniform values in vector registers: into scalar ones, so that the block's addresses are)
-    auto uni = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
-    const int run_s = uni(run), b0 = uni(run * R);
-    const AttnUnit un{uni(kh), uni(qg), run_s, b0, uni(min(nb, b0 + R))};
-    if (R == 1) attn_unit<NCH, I8, false>(q16, kvp, kvs, slots, nh, nkv, sp, parts, nb_max, G, un, lds_h, sc_l);
-    else attn_unit<NCH, I8, true>(q16, kvp, kvs, slots, nh, nkv, sp, parts, nb_max, G, un, lds_h, sc_l);
 }
 
 // The blocks joined per (row, head): exp(block max - max), the sums, 1 / sum, times sigmoid(gate)
@@ -530,7 +445,7 @@ __global__ __launch_bounds__(256, 2) void attn_block_kernel(const _Float16 *__re
 // a lane, and the waves' sums are added in order.
 __global__ __launch_bounds__(256) void attn_merge_kernel(const float *__restrict__ parts, const float *__restrict__ qkv,
                                                          int64_t ldq, int nh, int hd, int nb_max,
-                                                         const StepParams *__restrict__ sp, int nkv_groups,
+                                                         const StepParams *__restrict__ sp,
                                                          _Float16 *__restrict__ act, int64_t act_stride) {
     __shared__ float fw[1024];
     __shared__ float red[2][4];
@@ -538,7 +453,7 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(const float *__restrict
     trace(GV_K_MERGE, 0);
     const int t = blockIdx.x, h = blockIdx.y;
     if (t >= sp->M) return;
-    const int nbw = attn_runs(sp->pos + sp->M, nkv_groups);   // the partials of a (row, head)
+    const int nbw = (sp->pos + sp->M + kAttnBlock - 1) / kAttnBlock;
     const int ld = hd + 2;
     const float *base = parts + ((static_cast<int64_t>(t) * nh + h) * nb_max) * ld;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -583,7 +498,7 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(const float *__restrict
     for (int k = 0; k < 4; ++k) {
         const int bb = threadIdx.x + 256 * k;
         if (bb >= nbw) break;
-        const float f = bm[k] == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f(__fsub_rn(bm[k], mx));
+        const float f = bm[k] == -__builtin_inff() ? 0.0f : expf(__fsub_rn(bm[k], mx));
         fw[bb] = f;
         l = __builtin_fmaf(bs[k], f, l);
     }
@@ -656,7 +571,7 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(const float *__restrict
 // sixteen phases' sums are then added in a fixed order (lanes by xor 16 then 32, the waves in order).
 __global__ __launch_bounds__(256) void attn_merge64_kernel(const float *__restrict__ parts, const float *__restrict__ qkv,
                                                            int64_t ldq, int nh, int hd, int nb_max,
-                                                           const StepParams *__restrict__ sp, int nkv_groups,
+                                                           const StepParams *__restrict__ sp,
                                                            _Float16 *__restrict__ act, int64_t act_stride) {
     __shared__ float fw[1024];
     __shared__ float red[2][4];
@@ -664,7 +579,7 @@ __global__ __launch_bounds__(256) void attn_merge64_kernel(const float *__restri
     trace(GV_K_MERGE, 0);
     const int t = blockIdx.x, h = blockIdx.y, part = blockIdx.z;
     if (t >= sp->M) return;
-    const int nbw = attn_runs(sp->pos + sp->M, nkv_groups);   // the partials of a (row, head)
+    const int nbw = (sp->pos + sp->M + kAttnBlock - 1) / kAttnBlock;
     const int ld = hd + 2;
     const float *base = parts + ((static_cast<int64_t>(t) * nh + h) * nb_max) * ld;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, ph = 4 * wave + lane / 16, dq = lane % 16;
@@ -703,7 +618,7 @@ __global__ __launch_bounds__(256) void attn_merge64_kernel(const float *__restri
     for (int k = 0; k < 4; ++k) {
         const int bb = threadIdx.x + 256 * k;
         if (bb >= nbw) break;
-        const float f = bm[k] == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f(__fsub_rn(bm[k], mx));
+        const float f = bm[k] == -__builtin_inff() ? 0.0f : expf(__fsub_rn(bm[k], mx));
         fw[bb] = f;
         l = __builtin_fmaf(bs[k], f, l);
     }
@@ -1749,10 +1664,9 @@ int launch_attn_t(Model &m, LayerW &L, int M, hipStream_t st) {
     static int granted = 0;
     const size_t lds = attn_lds(NCH * 32);
     if (lds_grant(reinterpret_cast<const void *>(&attn_block_kernel<NCH, I8>), lds, granted) != 0) return -1;
-    // the units a step of M rows can have at any position, in whole eights when their groups go by XCD
-    const int G = attn_groups(c.n_heads, c.n_kv_heads, M), nkvg = c.n_kv_heads * G;
-    const int units = c.n_kv_heads * std::min(m.kv_blocks, (kAttnUnits + nkvg - 1) / nkvg);
-    const int grid = G == 1 ? units : (units + 7) / 8 * 8 * G;
+    // the units of any position, and the most that go in groups (in whole eights, by XCD)
+    const int G = attn_groups(c.n_heads, c.n_kv_heads, M), units = m.kv_blocks * c.n_kv_heads;
+    const int grid = G == 1 ? units : std::max(units, (std::min(units, kAttnGroupUnits * G) + 7) / 8 * 8 * G);
     hipLaunchKernelGGL((attn_block_kernel<NCH, I8>), dim3(grid), dim3(256), lds, st, m.q16,
                        I8 ? static_cast<const void *>(L.kv8) : static_cast<const void *>(L.kv), L.kvs, m.slots,
                        c.n_heads, c.n_kv_heads, m.sp, m.parts, m.kv_blocks, G);
@@ -1887,10 +1801,10 @@ int launch_class(Model &m, int cls, int l, int M, hipStream_t st) {
     case GV_K_MERGE:
         if (hd % 64 == 0)
             hipLaunchKernelGGL(attn_merge64_kernel, dim3(M, nh, hd / 64), dim3(256), 0, st, m.parts, m.qkv_out,
-                               L.qkv.rows, nh, hd, m.kv_blocks, m.sp, nkv * attn_groups(nh, nkv, M), m.act_core, abC);
+                               L.qkv.rows, nh, hd, m.kv_blocks, m.sp, m.act_core, abC);
         else
             hipLaunchKernelGGL(attn_merge_kernel, dim3(M, nh), dim3(256), 0, st, m.parts, m.qkv_out, L.qkv.rows, nh, hd,
-                               m.kv_blocks, m.sp, nkv * attn_groups(nh, nkv, M), m.act_core, abC);
+                               m.kv_blocks, m.sp, m.act_core, abC);
         return 0;
     case GV_K_O: {   // the residual add is the product's accumulate
         if (mixout) return launch_mixout(m, L, l, M, mix_kw, st);   // with the router and the route
