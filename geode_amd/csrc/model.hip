@@ -2855,7 +2855,7 @@ int stage_rows_in(Model &m, void *dst, const void *src, int64_t rows, size_t src
     GV_REQUIRE(step > 0, "gv_model_moe: a row wider than a staging slot");
     for (size_t o = 0; o < bytes; o += step) {
         const size_t n = std::min(step, bytes - o);
-        const int s = pf.stage_next++ % kStageSlots;
+        const int s = pf.stage_ring.take();
         char *slot = pf.stage + static_cast<size_t>(s) * kStageSlot;
         GV_CHECK_HIP(hipEventSynchronize(pf.stage_ev[s]));   // (its last copy done: at once for an event never recorded)
         if (plain) {
@@ -2897,7 +2897,7 @@ int stage_out(Model &m, const StagePiece *piece, int pieces, hipStream_t st) {
         for (size_t o = 0; o < piece[i].bytes; o += kStageSlot) {
             if (tail - head == kStageSlots && land() != 0) return -1;
             // (a slot still read by a copy in: the stream does that copy first)
-            const int s = pf.stage_next++ % kStageSlots;
+            const int s = pf.stage_ring.take();
             const size_t n = std::min(kStageSlot, piece[i].bytes - o);
             GV_CHECK_HIP(hipMemcpyAsync(pf.stage + static_cast<size_t>(s) * kStageSlot,
                                         static_cast<const char *>(piece[i].src) + o, n, hipMemcpyDeviceToHost, st));

@@ -11,6 +11,7 @@
 #include "../../include/geode_verify.h"
 #include "common.hpp"
 #include "kernels.hpp"
+#include "ring.hpp"
 
 namespace gv {
 
@@ -87,6 +88,9 @@ struct LayerW {
     float *c_slots = nullptr;     // [2 max_rows][K - 1][conv_dim] conv states
 };
 
+constexpr int kStageSlots = 8;   // gv_model_moe's staging slots, and the bytes of one
+constexpr size_t kStageSlot = size_t{1} << 20;
+
 // The prefill MoE's buffers (C5: many rows), allocated for `cap` rows on first use
 struct Prefill {
     int cap = 0, M = 0, layer = 0;   // M, layer: the last gv_model_moe call's (for the replay)
@@ -100,11 +104,9 @@ struct Prefill {
     // gv_model_moe's rows on their way between the caller's memory and the device: pinned slots used in turn, an event
     // a slot (allocated on the first call, given back with the model)
     char *stage = nullptr;
-    hipEvent_t stage_ev[8] = {};
-    int stage_next = 0;
+    hipEvent_t stage_ev[kStageSlots] = {};
+    Ring<kStageSlots> stage_ring;
 };
-constexpr int kStageSlots = 8;
-constexpr size_t kStageSlot = size_t{1} << 20;
 
 struct Model {
     gv_model_config c{};
