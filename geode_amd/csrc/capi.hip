@@ -296,13 +296,17 @@ int ffn_swiglu_ws(const gv_q4 *gate, const gv_q4 *up, const gv_q4 *down, int M, 
     const int64_t ab_h = act_halves(H), ab_f = act_halves(F);
     if (H <= 8192 && (M <= 8 || F <= 8192) && ffn_up_fits(to_q4(*gate), to_q4(*up), M)) {
         // x's operands (in x's place: M act rows of H fit its M x H floats), gate | up with the SwiGLU and its
-        // quantization (act), down. Wider inputs than the gate | up launch's eight waves take go on below, in a launch
-        // a phase (17 rows of 2048 -> 6144: 58 us a call that way, 30 this one).
+        // quantization (act), down. Inputs wider than the gate | up launch's eight waves take, and more than 8 rows
+        // of an ff beyond 8192, go on below, in a launch a phase (17 rows of 2048 -> 6144: 58 us a call that way, 30 this
+        // one).
         _Float16 *act_x = reinterpret_cast<_Float16 *>(x);
         if (quantize_f16(x_f16, M, static_cast<int>(H), act_x, ab_h, st) != 0) return -1;
         if (ffn_up(to_q4(*gate), to_q4(*up), act_x, ab_h, M, act, ab_f, st) != 0) return -1;
         return gemv_q4(to_q4(*down), act, ab_f, M, gemv_out(y, H, down->global), st);
     }
+    // (these launches' operands: rows of at most 8192 values; refused here, before the first of them writes to ws)
+    GV_REQUIRE(H <= 8192 && F <= 8192, "gv_ffn_swiglu: hidden and ff at most 8192 (ff up to 16384: at most 8 rows, hidden "
+                                       "within the fused launch's eight waves)");
     if (f16_to_f32(x_f16, static_cast<int64_t>(M) * H, x, st) != 0) return -1;
     if (quantize_act(x, H, M, static_cast<int>(H), nullptr, 0.0f, act, ab_h, nullptr, 0, st) != 0) return -1;
     if (gemv_q4(to_q4(*gate), act, ab_h, M, gemv_out(g, F, gate->global), st) != 0) return -1;

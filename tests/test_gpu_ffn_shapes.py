@@ -41,6 +41,29 @@ def test_ffn_shapes(gv, H, F, M):
     assert np.abs(got - exact).max() <= 1.5 * np.abs(want - exact).max() + 1e-6 * np.abs(exact).max()
 
 
+@pytest.mark.parametrize("H,F,M,taken", [(2048, 8448, 8, True), (2048, 8448, 9, False), (2048, 8192, 9, True)])
+def test_ffn_width_limit(gv, H, F, M, taken):
+    """ff beyond 8192: up to 8 rows; more rows are refused before anything is launched (the workspace and the output as
+    they were)."""
+    gq, gg = po.q4_random(1001, F, H)
+    dq, dg = po.q4_random(1003, H, F)
+    x16 = po.f32_to_f16_bits(po.normal(2001, M * H).reshape(M, H))
+    G, D = gv.Q4Matrix(gq, F, H, gg), gv.Q4Matrix(dq, H, F, dg)
+    dx = gv.DeviceBuffer.from_array(x16)
+    n = gv.lib.gv_ffn_workspace_bytes(H, F, M) // 4
+    y, ws = (gv.DeviceBuffer.from_array(np.full(k, 7.0, np.float32)) for k in (M * H, n))
+    rc = gv.lib.gv_ffn_swiglu(G.ref(), G.ref(), D.ref(), M, dx.ptr, y.ptr, ws.ptr)
+    gv.check(gv.lib.gv_synchronize(), "synchronize")
+    got = y.download(np.float32, (M, H))
+    if taken:
+        want = po.ffn_swiglu(gq, gq, dq, gg, gg, dg, H, F, x16, mode=0)
+        # (test_ffn_shapes' bound, a row's)
+        assert rc == 0 and np.abs(got - want).max() <= 1e-2 * np.abs(want).max()
+    else:
+        assert rc != 0 and b"at most 8192" in gv.lib.gv_last_error()
+        assert np.all(got == 7.0) and np.all(ws.download(np.float32, (n,)) == 7.0)
+
+
 @pytest.mark.parametrize("rows,cols,M", [(2048, 6144, 1), (600, 6144, 8), (16, 4608, 3), (600, 6144, 17),
                                          (600, 2048, 17), (2048, 1152, 32), (4096, 4096, 31), (40, 128, 20),
                                          (2100, 2048, 17), (4112, 4608, 8)])
