@@ -335,7 +335,8 @@ __device__ inline void mfma_tiles_of(const MatFn mat, int64_t rows, int nsc, int
     static_assert(DEPTH >= 2 && (NT > 0 || DEPTH >= 3), "the runtime loop is a ring of at least three");
     static_assert(PACK <= 1 || NTT == 2, "packed after a whole tile: two tiles, at most 24 rows");
     static_assert(PACK != 1 || NTT == 1, "packed hi | lo columns take one 16-row tile of at most 8 rows");
-    static_assert(BUFS == 1 || FLUSH > 0, "turns are of the flushed tiles");
+    static_assert(BUFS == 1 || (FLUSH > 0 && FlushFn::active),
+                  "two halves in turn: flushed tiles, by a flush of the call's own (put's epilogue reads the first half only)");
     static_assert(FLUSH == 0 || (MODE == kSplitK && NT == 0), "the flushed split-K runs the runtime tile loop");
     constexpr int NB = PACK == 1 ? 1 : 2;   // operand arrays: hi | lo packed, or hi and lo
     constexpr auto packed = [](int tt) { return PACK == 1 || (PACK == 2 && tt == 1); };   // (column tile tt)
