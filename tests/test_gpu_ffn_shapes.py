@@ -1,6 +1,7 @@
 """The dense MLP and the skinny product where their launches change form: rows at the edges of the 8-, 16- and 32-row
 forms, K ranges of one launch and of several (12 waves at K 4608..6144 and at most 256 row tiles, row groups at 17..32
-rows over few tiles), ragged last row tiles, against the CPU oracle's int8 path."""
+rows over few tiles, both K ranges of 4096 in one launch over more), ragged last row tiles, against the CPU oracle's int8
+path."""
 import numpy as np
 import pytest
 
@@ -66,7 +67,7 @@ def test_ffn_width_limit(gv, H, F, M, taken):
 
 @pytest.mark.parametrize("rows,cols,M", [(2048, 6144, 1), (600, 6144, 8), (16, 4608, 3), (600, 6144, 17),
                                          (600, 2048, 17), (2048, 1152, 32), (4096, 4096, 31), (40, 128, 20),
-                                         (2100, 2048, 17), (4112, 4608, 8)])
+                                         (2100, 2048, 17), (4112, 4608, 8), (4112, 4096, 17), (8192, 4096, 32)])
 @pytest.mark.parametrize("accumulate", [False, True])
 def test_gemv_few_tiles(gv, rows, cols, M, accumulate):
     wq, s2 = po.q4_random(31 + rows + cols, rows, cols)
