@@ -633,8 +633,10 @@ int gemv_q4(const Q4 &w, const _Float16 *act, int64_t act_stride, int M, const G
     if (M <= 8 && nsc > 32 && nsc <= 48 && nsc % 4 == 0 && ntiles <= 256) {
         // K of 4096 .. 6144 over at most a tile a CU (a dense MLP's down product): one launch of up to twelve waves,
         // 512 values each, instead of two K ranges one after the other - with a tile a workgroup a launch is one
-        // round of loads, so the second range's launch costs as much as the first's. More tiles (each CU streaming
-        // many) or wider K (the waves' operands no longer fit their registers): the ranges below.
+        // round of loads, so the second range's launch costs about as much as the first's. 2048 rows, 5 rows of x: K =
+        // 4608 6.7 us (4352, in ranges: 7.2 + 3.7), 6144 7.8 us (5888, in ranges: 7.1 + 4.7). A wave takes 512 values, so
+        // K in multiples of it; 9..16 rows (unpacked: twice the operand registers, which twelve waves do not have; 9 rows
+        // at 6144: 9.4 + 6.1), more tiles (each CU streaming many) or wider K: the ranges below.
         const int waves = nsc / 4;
         hipLaunchKernelGGL((gemv_q4_kernel<16, 1, 12, true, 1>), dim3(static_cast<unsigned>(ntiles)),
                            dim3(64 * waves), static_cast<size_t>(waves) * 1024, st, w, act, act_stride, M, 0, 1, out);
